@@ -199,6 +199,7 @@ __device__ void softmax_requant_rows(const float* s, const float* row_max, float
 extern "C" __global__ void __launch_bounds__(256) mxfa_softmax_requant_rows(
     const float* s, const float* row_max, float c, int64_t rows, int cols, float* p, uint8_t* codes,
     uint8_t* scales, float* row_sum, int p_rule) {
+  fp8_saturate();
   if (p_rule == P_R2)
     softmax_requant_rows<P_R2>(s, row_max, c, rows, cols, p, codes, scales, row_sum);
   else
@@ -416,11 +417,6 @@ __device__ __forceinline__ float in_vgpr(float x) {
   __asm__("v_mov_b32 %0, %1" : "=v"(r) : "s"(x));
   return r;
 }
-__device__ __forceinline__ uint32_t in_vgpr_u(uint32_t x) {
-  uint32_t r;
-  __asm__("v_mov_b32 %0, %1" : "=v"(r) : "s"(x));
-  return r;
-}
 
 // fp32 subnormal results flushed to zero (MODE.FP_DENORM single-precision bits = 0) for the
 // rest of the wave.  The pipelined prefill kernels rely on it for the R1 flush of P (below);
@@ -440,10 +436,8 @@ __device__ __forceinline__ float pair_max_raw(float x) {
 // applies (y < 2^-126), and no exponential lands in between: sc <= 119 (amax <= 1), so
 // P = exp2(x) with x within 2^-19 of an integer e <= -14 is 2^e itself or at least ~10 ulps
 // from it.  The kept values convert as y * 2^120 = P / 2^(sc - 127), the same codes.
-__device__ __forceinline__ uint32_t p_pack4_ftz(float y0, float y1, float y2, float y3, uint32_t ones) {
-  const uint32_t w = cvt_pack4_in_place(y0, y1, y2, y3, __uint_as_float(7u << 23));   // 2^-120
-  const uint32_t top = (w + ones) >> 7;               // bit 0 of each byte: that byte was 0x7f
-  return w ^ (top & ones);                            // 0x7f -> 0x7e, other bytes unchanged
+__device__ __forceinline__ uint32_t p_pack4_ftz(float y0, float y1, float y2, float y3) {
+  return cvt_pack4_in_place(y0, y1, y2, y3, __uint_as_float(7u << 23));   // 2^-120
 }
 
 __device__ __forceinline__ float vmin(float a, float b) { return __builtin_elementwise_minimum(a, b); }
@@ -515,10 +509,8 @@ __device__ __forceinline__ void pipe_softmax(float& m, float& l, v16f (&s)[BN / 
 #pragma unroll
       for (int i = 0; i < 16; i++) p[i] = __builtin_amdgcn_exp2f(arg(s[t][i]));
       const float f = __uint_as_float((134u - sc) << 23);     // 2^(7 - sc)
-      const uint32_t ones = in_vgpr_u(0x01010101u);
 #pragma unroll
-      for (int g = 0; g < 4; g++)
-        w[g] = p_pack4_ftz(p[4 * g] * f, p[4 * g + 1] * f, p[4 * g + 2] * f, p[4 * g + 3] * f, ones);
+      for (int g = 0; g < 4; g++) w[g] = p_pack4_ftz(p[4 * g] * f, p[4 * g + 1] * f, p[4 * g + 2] * f, p[4 * g + 3] * f);
     }
     // row-sum terms (every P, including those R1 flushes from the codes) in four
     // independent chains (no 32-deep add dependency)

@@ -37,6 +37,7 @@ __device__ void decode_split_impl(const FaArgs& a) {
   // contiguous 1 KB row, so that a block's K and V codes stay in flight in registers
   constexpr bool QLDS = D == 256;
   __shared__ __attribute__((aligned(16))) v4i sQ[QLDS ? NW : 1][QLDS ? D / 16 * 64 : 1];
+  fp8_saturate();                                     // the P codes' saturation
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
   // one (batch, KV head, chunk) item per wave, items numbered chunk-fastest over the
