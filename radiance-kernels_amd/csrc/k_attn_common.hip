@@ -199,7 +199,6 @@ __device__ void softmax_requant_rows(const float* s, const float* row_max, float
 extern "C" __global__ void __launch_bounds__(256) mxfa_softmax_requant_rows(
     const float* s, const float* row_max, float c, int64_t rows, int cols, float* p, uint8_t* codes,
     uint8_t* scales, float* row_sum, int p_rule) {
-  fp8_saturate();
   if (p_rule == P_R2)
     softmax_requant_rows<P_R2>(s, row_max, c, rows, cols, p, codes, scales, row_sum);
   else
@@ -417,6 +416,11 @@ __device__ __forceinline__ float in_vgpr(float x) {
   __asm__("v_mov_b32 %0, %1" : "=v"(r) : "s"(x));
   return r;
 }
+__device__ __forceinline__ uint32_t in_vgpr_u(uint32_t x) {
+  uint32_t r;
+  __asm__("v_mov_b32 %0, %1" : "=v"(r) : "s"(x));
+  return r;
+}
 
 // fp32 subnormal results flushed to zero (MODE.FP_DENORM single-precision bits = 0) for the
 // rest of the wave.  The pipelined prefill kernels rely on it for the R1 flush of P (below);
@@ -430,14 +434,41 @@ __device__ __forceinline__ float pair_max_raw(float x) {
   return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// MODE.FP16_OVFL between sat_begin and sat_end: a conversion to fp8 whose rounded result is above
+// 448 returns 0x7e instead of the NaN code 0x7f (every other code unchanged, NaN included), so
+// the packed codes need no fix -- three instructions per four codes, 24 of the prefill's 317 VALU
+// instructions per 32 queries x 64 keys, and the prefill is bound by VALU issue (B = 2, Hq 32, S =
+// 4096, D = 128: 260.2 -> 253.0 us; D = 256 with softcap and window, S = 8192: 435.2 -> 428.2).
+// The bit must not be set while an MFMA issues: it would also turn infinite and NaN
+// results into finite ones.  The operands order the instructions: every exponential of the block
+// reads the value that sat_begin returns, which depends on every score; sat_end reads the codes,
+// and PV the scale that it returns: no MFMA can issue inside the window.  (The row sum passes
+// through sat_end so that its terms die inside the window too; left behind it they spilled.)
+// The workspace-free softcap kernels at D = 256, at their register limit, keep the packed fix
+// (HS = false): the window spills 9 registers there (Hq 16, S = 4096: 214.5 against 194.3 us).
+__device__ __forceinline__ void sat_begin(float& mcn) {
+  __asm__ volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1" : "+v"(mcn));
+}
+__device__ __forceinline__ void sat_end(const v8i& w, int& sc, float& l) {
+  __asm__ volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 0"
+                   : "+v"(sc), "+v"(l)
+                   : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]));
+}
+
 // R1 codes of four P values of a tile with scale code sc, given y = P * 2^(7 - sc) computed
 // with fp32 subnormals flushed (fp32_flush_denormals): the R1 flush bound of the tile,
 // F4M3 * 2^(sc - 127), is within two ulps below 2^(sc - 133), the bound that the flush to zero
 // applies (y < 2^-126), and no exponential lands in between: sc <= 119 (amax <= 1), so
 // P = exp2(x) with x within 2^-19 of an integer e <= -14 is 2^e itself or at least ~10 ulps
-// from it.  The kept values convert as y * 2^120 = P / 2^(sc - 127), the same codes.
-__device__ __forceinline__ uint32_t p_pack4_ftz(float y0, float y1, float y2, float y3) {
-  return cvt_pack4_in_place(y0, y1, y2, y3, __uint_as_float(7u << 23));   // 2^-120
+// from it.  The kept values convert as y * 2^120 = P / 2^(sc - 127), the same codes.  R1's
+// saturation at 448 is the conversion's own between sat_begin and sat_end (HS), else a fix of the
+// packed codes.
+template <bool HS>
+__device__ __forceinline__ uint32_t p_pack4_ftz(float y0, float y1, float y2, float y3, uint32_t ones) {
+  const uint32_t w = cvt_pack4_in_place(y0, y1, y2, y3, __uint_as_float(7u << 23));   // 2^-120
+  if constexpr (HS) return w;
+  const uint32_t top = (w + ones) >> 7;               // bit 0 of each byte: that byte was 0x7f
+  return w ^ (top & ones);                            // 0x7f -> 0x7e, other bytes unchanged
 }
 
 __device__ __forceinline__ float vmin(float a, float b) { return __builtin_elementwise_minimum(a, b); }
@@ -460,7 +491,7 @@ __device__ __forceinline__ float pair_min_raw(float x) {
 // -inf for a fully masked tile (cap2 * inf).
 // VG: the softcap constants in VGPRs (full-rate VALU at three waves per SIMD); at two waves
 // per SIMD SGPR operands cost nothing and save the registers.
-template <bool SOFTCAP, int PR, bool VG = true>
+template <bool SOFTCAP, int PR, bool VG = true, bool HS = true>
 __device__ __forceinline__ void pipe_softmax(float& m, float& l, v16f (&s)[BN / 32],
                                              v8i& pb, int (&psc)[BN / 32], float& corr, float c,
                                              float cap2 = 0.0f, float cap = 0.0f) {
@@ -480,7 +511,8 @@ __device__ __forceinline__ void pipe_softmax(float& m, float& l, v16f (&s)[BN / 
   const float mu = m_new == -INFINITY ? 0.0f : m_new;
   corr = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mu) * c);
   m = m_new;
-  const float mcn = SOFTCAP ? cap - mu : -(mu * c);
+  float mcn = SOFTCAP ? cap - mu : -(mu * c);
+  if constexpr (PR != P_R2 && HS) sat_begin(mcn);
   auto arg = [&](float x) { return SOFTCAP ? __builtin_fmaf(cap2, x, mcn) : __builtin_fmaf(x, c, mcn); };
   float part[4];
 #pragma unroll
@@ -509,8 +541,10 @@ __device__ __forceinline__ void pipe_softmax(float& m, float& l, v16f (&s)[BN / 
 #pragma unroll
       for (int i = 0; i < 16; i++) p[i] = __builtin_amdgcn_exp2f(arg(s[t][i]));
       const float f = __uint_as_float((134u - sc) << 23);     // 2^(7 - sc)
+      const uint32_t ones = in_vgpr_u(0x01010101u);     // (HS = false only)
 #pragma unroll
-      for (int g = 0; g < 4; g++) w[g] = p_pack4_ftz(p[4 * g] * f, p[4 * g + 1] * f, p[4 * g + 2] * f, p[4 * g + 3] * f);
+      for (int g = 0; g < 4; g++)
+        w[g] = p_pack4_ftz<HS>(p[4 * g] * f, p[4 * g + 1] * f, p[4 * g + 2] * f, p[4 * g + 3] * f, ones);
     }
     // row-sum terms (every P, including those R1 flushes from the codes) in four
     // independent chains (no 32-deep add dependency)
@@ -520,6 +554,7 @@ __device__ __forceinline__ void pipe_softmax(float& m, float& l, v16f (&s)[BN / 
     for (int g = 0; g < 4; g++) pb[4 * (t & 1) + g] = (int)w[g];
   }
   l = l * corr + ((part[0] + part[1]) + (part[2] + part[3]));
+  if constexpr (PR != P_R2 && HS) sat_end(pb, psc[0], l);
 }
 // Score post-processing of one block in place: softcap (log2 units), then the mask.
 // softcap * tanh(u), u = s * scale / softcap, in log2 units: cap_log2 * (1 - 2 / (e + 1)) =

@@ -296,7 +296,6 @@ __device__ void prefill3_impl(const FaArgs& a) {
   using L = P3Lds<D>;
   constexpr int NW = P3Waves<D>::N;
   fp32_flush_denormals();   // pipe_softmax's R1 flush
-  fp8_saturate();           // and its saturation
   constexpr bool K1 = NOWS || p3_one_k_stage<D>();
   __shared__ __attribute__((aligned(16))) uint8_t sKb0[L::KB];
   __shared__ __attribute__((aligned(16))) uint8_t sKb1[K1 ? 16 : L::KB];
@@ -439,7 +438,7 @@ __device__ void prefill3_impl(const FaArgs& a) {
     v8i pb;
     int psc[BN / 32];
     float corr;
-    pipe_softmax<SOFTCAP, PR, D <= 128>(m, l, sc, pb, psc, corr, c, -2.0f * a.cap_log2, a.cap_log2);
+    pipe_softmax<SOFTCAP, PR, D <= 128, !(NOWS && SOFTCAP && D == 256)>(m, l, sc, pb, psc, corr, c, -2.0f * a.cap_log2, a.cap_log2);
     if constexpr (TRACE) {
       const float lrow = pair_sum(l);
       if (traced) {

@@ -168,19 +168,13 @@ __device__ __forceinline__ uint32_t e3m2x4_to_e4m3x4(uint32_t w) {
 // 2^-126) reaches it.  The conversion then divides by its scale operand; it uses only that
 // operand's exponent field (measured on gfx950: 1.5 acts as 1, 3.0 as 2, and a float with
 // exponent field 0 as 2^-127), so (sc << 23) | 0x400000 is 2^(sc - 127) for every code,
-// sc = 0 included.  The 448 saturation is the conversion's own: the kernels that call these
-// routines set MODE.FP16_OVFL first (fp8_saturate).
+// sc = 0 included.  The 448 saturation is applied to the packed codes: the conversion has
+// no saturating form and returns 0x7f for a scaled value above 464 (values in (448, 464]
+// round to 448); a P never exceeds its tile amax by more than a rounding residue and the
+// amax scales into [256, 512), so every code is at most 0x7f and 0x7f -> 0x7e is exactly
+// R1's saturation (three instructions per four codes instead of a min per value).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kE4M3FlushBits = (120u << 23) | 0x7ffffeu;   // F4M3
-
-// MODE.FP16_OVFL = 1 for the rest of the wave: a conversion to fp8 whose rounded result is above
-// 448 (or infinite) returns +-448 (0x7e / 0xfe) instead of 0x7f / 0xff; every other code and NaN
-// are unchanged (checked on every float in [400, 600) and a stride over all others, at the scales 1, 2^-60
-// and 2^-120).  The packed-byte fix it replaces was 24 of the prefill's 317 VALU instructions per
-// 32 queries x 64 keys.
-__device__ __forceinline__ void fp8_saturate() {
-  __builtin_amdgcn_s_setreg((0 << 11) | (23 << 6) | 1, 1);   // hwreg(MODE, 23, 1)
-}
 
 struct PTileBounds {
   float flush, scale;
@@ -223,7 +217,9 @@ __device__ __forceinline__ uint32_t cvt_pack4_in_place(float y0, float y1, float
 // Four P values (>= 0, finite, at most the tile amax) of one tile -> their R1 E4M3 codes
 // (byte i = value i).
 __device__ __forceinline__ uint32_t p_pack4(float p0, float p1, float p2, float p3, const PTileBounds& b) {
-  return cvt_pack4_in_place(p_flush(p0, b), p_flush(p1, b), p_flush(p2, b), p_flush(p3, b), b.scale);
+  const uint32_t w = cvt_pack4_in_place(p_flush(p0, b), p_flush(p1, b), p_flush(p2, b), p_flush(p3, b), b.scale);
+  const uint32_t top = (w + 0x01010101u) >> 7;     // bit 0 of each byte: that byte was 0x7f
+  return w ^ (top & 0x01010101u);                  // 0x7f -> 0x7e, other bytes unchanged
 }
 
 // R1 E4M3 codes of four already scaled values of any sign (byte i = value i), on the
