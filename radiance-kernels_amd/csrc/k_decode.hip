@@ -327,29 +327,30 @@ MXFA_DECODE_ALL(128)
 MXFA_DECODE_ALL(256)
 
 // Merge nparts partials per (b, query head): O = sum_i O_i 2^{(m_i - M) c} / sum_i l_i 2^{(m_i - M) c}.
-// One workgroup per (query head, 64 columns): 16 lanes hold the 64 columns of one partial (256
-// contiguous bytes), group g = tid / 16 of the workgroup takes the partials g, g + ngrp, ... in
-// order, CU of them in flight (their loads issued before the maximum is known), and the groups'
-// sums are added in group order.  At most 4 partials are one group's work: then every product
-// is added in part order by one chain of fmas, bit for bit the merge inside the decode
-// workgroup.  The merge is latency: one thread walking the partials with two dependent loads
-// each took 97 us for 256 partials of 32 heads (one sequence of 131,072 keys) and 10 us for 24
-// of 128; this form 4.7 and 3.4 us.
+// 16 lanes hold 64 columns of one partial (256 contiguous bytes).  One workgroup per (query head, 64
+// columns); group g = tid / 16 takes the partials g, g + ngrp, ... in order, CB_U of them in
+// flight (their loads issued before the maximum is known), and the groups' sums are added in
+// group order.  Up to 4 partials one workgroup per query head instead, each group one 64-column
+// slice and all partials: every product is then added in part order by one chain of fmas, bit
+// for bit the merge inside the decode workgroup.  The merge is latency: one thread per column
+// walking the partials with two dependent loads each took 97 us for 256 partials of 32 heads
+// (one sequence of 131,072 keys), 11.9 us for 24 of 128; this form 5.6 and 4.0 us.
 constexpr int CB_U = 4;
 
-extern "C" __global__ void __launch_bounds__(1024) mxfa_decode_combine(FaArgs a) {
-  __shared__ float smax[16];
-  __shared__ float sl[64];
-  __shared__ __attribute__((aligned(16))) float so[64][64];
+extern "C" __global__ void __launch_bounds__(512) mxfa_decode_combine(FaArgs a) {
+  __shared__ float smax[8];
+  __shared__ float sl[32];
+  __shared__ __attribute__((aligned(16))) float so[32][64];
   const int64_t bh = blockIdx.x;
-  const int D = 64 * (int)gridDim.y;
   const int nparts = a.n_qblk;
+  const bool serial = nparts <= 4;                   // (the launch's shape follows the same rule)
+  const int D = serial ? 4 * (int)blockDim.x : 64 * (int)gridDim.y;
   const float c = a.cap_log2 > 0.0f ? 1.0f : a.c_log2;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int grp = tid >> 4, col = 4 * (tid & 15);
-  const int ngrp = nparts <= 4 ? 1 : (int)blockDim.x >> 4;
+  const int grp = serial ? 0 : tid >> 4, ngrp = serial ? 1 : (int)blockDim.x >> 4;
+  const int d = serial ? 4 * tid : 64 * (int)blockIdx.y + 4 * (tid & 15);
   const float2* ml = reinterpret_cast<const float2*>(a.part_ml) + bh * nparts;
-  const float* po = a.part_o + bh * nparts * D + 64 * blockIdx.y + col;
+  const float* po = a.part_o + bh * nparts * D + d;
   float2 x[CB_U];
   float4 o[CB_U];
   // partials i0 + u ngrp, clamped to the last one (whose repeats carry no weight)
@@ -363,18 +364,20 @@ extern "C" __global__ void __launch_bounds__(1024) mxfa_decode_combine(FaArgs a)
   };
   load(grp);
   float M = -INFINITY;
-  for (int i = tid; i < nparts; i += blockDim.x) {
+  for (int i = serial ? 0 : tid; i < nparts; i += serial ? 1 : blockDim.x) {
     const float2 y = ml[i];
     if (y.y > 0.0f) M = fmaxf(M, y.x);
   }
+  if (!serial) {
 #pragma unroll
-  for (int k = 1; k < 64; k <<= 1) M = fmaxf(M, __shfl_xor(M, k));
-  if (lane == 0) smax[tid >> 6] = M;
-  __syncthreads();
-  for (int w = 0; w < (int)blockDim.x >> 6; w++) M = fmaxf(M, smax[w]);
+    for (int k = 1; k < 64; k <<= 1) M = fmaxf(M, __shfl_xor(M, k));
+    if (lane == 0) smax[tid >> 6] = M;
+    __syncthreads();
+    for (int w = 0; w < (int)blockDim.x >> 6; w++) M = fmaxf(M, smax[w]);
+  }
   float L = 0.0f;
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (M != -INFINITY && grp < ngrp) {
+  if (M != -INFINITY) {
     const float mc = M * c;
     for (int i0 = grp; i0 < nparts; i0 += CB_U * ngrp) {
       if (i0 != grp) load(i0);
@@ -391,10 +394,14 @@ extern "C" __global__ void __launch_bounds__(1024) mxfa_decode_combine(FaArgs a)
       }
     }
   }
-  if (grp < ngrp) {
-    *reinterpret_cast<float4*>(&so[grp][col]) = acc;
-    if ((tid & 15) == 0) sl[grp] = L;
+  if (serial) {
+    const bool any = L > 0.0f;
+    *reinterpret_cast<float4*>(a.o + bh * D + d) = make_float4(any ? acc.x / L : 0.0f, any ? acc.y / L : 0.0f,
+                                                               any ? acc.z / L : 0.0f, any ? acc.w / L : 0.0f);
+    return;
   }
+  *reinterpret_cast<float4*>(&so[grp][4 * (tid & 15)]) = acc;
+  if ((tid & 15) == 0) sl[grp] = L;
   __syncthreads();
   if (tid < 64) {
     float s = so[0][tid], lt = sl[0];

@@ -711,10 +711,15 @@ mxfa_status decode_launch(DeviceModule* dm, const mxfa_attn_params* p, const uin
                               stream))
     return st;
   if (a.fuse_combine) return MXFA_OK;
-  // 16 partials of a head at a time, or 64 when there are more than 64: measured on 256 partials
-  // of 32 heads (D = 128) @@
-  return launch(dm, "mxfa_decode_combine", dim3((unsigned)nbh, (unsigned)(p->head_dim / 64)), dim3(nparts > 64 ? 1024 : 256),
-                args, stream);
+  // Groups of 16 threads per workgroup of the merge: 4 up to 32 partials, where more threads
+  // cost more than their partials in flight give (24 partials of 128 heads 4.0 us against 4.1 with
+  // 16 groups and 5.0 with 64; 16 partials of 2,048 heads 6.2, 8.6 and 28), then 16 (64 partials of
+  // 128 heads 3.3 against 4.5 with 4) and above 128 partials 32 (256 of 32 heads 5.2 against
+  // 11.2 and 6.0 with 4 and 16).
+  if (nparts <= 4)
+    return launch(dm, "mxfa_decode_combine", dim3((unsigned)nbh), dim3((unsigned)(p->head_dim / 4)), args, stream);
+  return launch(dm, "mxfa_decode_combine", dim3((unsigned)nbh, (unsigned)(p->head_dim / 64)),
+                dim3(nparts <= 32 ? 64 : nparts <= 128 ? 256 : 512), args, stream);
 }
 
 }  // namespace

@@ -27,10 +27,10 @@ def test_nan_key_code_reaches_every_row_that_sees_it(D, softcap, ws):
     assert bool(nan[:, 128:].all()) and bool(torch.isfinite(o[0, :, :100]).all())
 
 
-@pytest.mark.parametrize("parts", [4, 5, 16, 17, 63, 64, 65, 255, 257, 300])
+@pytest.mark.parametrize("parts", [4, 5, 16, 17, 32, 33, 128, 129, 257, 300])
 def test_decode_merge_part_counts(monkeypatch, parts):
-    """mxfa_decode_combine at the edges of its part groups: one group up to 4 partials, 16 or 64
-    groups above, with and without a remainder, and a last batch partly past the end."""
+    """mxfa_decode_combine at the edges of its part groups: one up to 4 partials, then 4, 16 and 32
+    groups, with and without a remainder, and a last batch partly past the end."""
     L = 64 * 300 + 32
     monkeypatch.setenv("MXFA_DECODE_WAVES", str(parts))
     monkeypatch.setenv("MXFA_DECODE_COMBINE", "kernel")
