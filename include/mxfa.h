@@ -142,6 +142,10 @@ mxfa_status mxfa_prefill(const mxfa_attn_params *p,
  * inputs, outputs and O as mxfa_prefill (bit-identical with E4M3 V, where both run the same
  * arithmetic in the same order; within a few ulps with E3M2 V).  Block-packed E3M2 V needs no
  * copy: the kernel reads it from v as it is.
+ * Calls with too few query rows to fill the chip and a long key range (1,024 visible keys or more,
+ * and at most 32 query rows or more than 5,120 keys) split the range: the workspace then holds
+ * partial results, and O differs from mxfa_prefill's by the order of fp32 additions (rel-L2 below
+ * 1e-6; the P codes are the same).
  * *workspace_bytes = batch * num_kv_heads * seq_k * head_dim * (2, or 3 with MXFA_FMT_E3M2 V).  A
  * workspace smaller than the plan is MXFA_ERR_WORKSPACE.
  * Replaces the same reference entry point as mxfa_prefill (kernels/flash_attention_mx_gqa/
@@ -158,7 +162,7 @@ mxfa_status mxfa_prefill_ws(const mxfa_attn_params *p,
 /* Test entry (V as E4M3 or E3M2 codes): the stages of the workspace prefill for query rows 32 * q_tile .. + 31 of head bh
  * (= batch * num_q_heads + query head), as its own routines compute them.  Runs the one
  * workgroup of mxfa_prefill_ws that holds those rows (writing their O rows, bit-identical to
- * mxfa_prefill_ws) and records, for each key block the workgroup processes:
+ * mxfa_prefill_ws where that does not split the key range) and records, for each key block the workgroup processes:
  *   s_out  [32][seq_k]        scores after softcap and mask (-inf masked); units: the raw
  *                             dot product q.k without softcap, softcap * tanh(.) * log2(e) with
  *   ml_out [ceil(seq_k/64)][32][2]  running max (same units) and row sum after the block

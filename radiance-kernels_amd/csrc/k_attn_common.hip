@@ -674,10 +674,11 @@ __device__ __forceinline__ void pv_parts_blk(v16f (&o)[D / 32], const uint8_t* s
 // writes.  Per 64-column chunk the wave writes its 32 x 64 floats to its private 8 KB slice
 // ldsw (the 16-byte chunk c of row r at c ^ (r & 15)), then reads 4 rows x 256 contiguous
 // bytes per instruction and stores them non-temporally (O is not read again here, so K and V
-// keep the L2).  Rows qw0 + row >= Sq are not stored.
-template <int D>
+// keep the L2).  Rows qw0 + row >= Sq are not stored.  rstride: floats between rows (D, or more for
+// the partials of a split prefill, which are read again).
+template <int D, bool NT = true>
 __device__ __forceinline__ void store_o_lds(const v16f (&o)[D / 32], float inv, float* ldsw, float* obase, int qw0,
-                                            int Sq, int lane) {
+                                            int Sq, int lane, int rstride = D) {
   const int r = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int p = 0; p < D / 64; p++) {
@@ -694,9 +695,11 @@ __device__ __forceinline__ void store_o_lds(const v16f (&o)[D / 32], float inv, 
     for (int k = 0; k < 8; k++) {
       const int row = 4 * k + (lane >> 4), c = lane & 15;
       const float4 v = *reinterpret_cast<const float4*>(ldsw + row * 64 + ((c ^ (row & 15)) << 2));
-      if (qw0 + row < Sq)
-        __builtin_nontemporal_store(__builtin_bit_cast(v4i, v),
-                                    reinterpret_cast<v4i*>(obase + (int64_t)(qw0 + row) * D + 64 * p + 4 * c));
+      if (qw0 + row < Sq) {
+        v4i* const dst = reinterpret_cast<v4i*>(obase + (int64_t)(qw0 + row) * rstride + 64 * p + 4 * c);
+        if constexpr (NT) __builtin_nontemporal_store(__builtin_bit_cast(v4i, v), dst);
+        else *dst = __builtin_bit_cast(v4i, v);
+      }
     }
   }
 }

@@ -286,12 +286,23 @@ __device__ __forceinline__ int fresh_lane() {
   return l;
 }
 
+// Key range ks of the nsplit that a split call cuts a workgroup's key blocks [j0, j1) into (of equal
+// length, the last ones shorter or empty).
+__device__ __forceinline__ void split_range(const FaArgs& a, int ks, int& j0, int& j1) {
+  const int len = (j1 - j0 + a.nsplit - 1) / a.nsplit;
+  j0 = min(j1, j0 + ks * len);
+  j1 = min(j1, j0 + len);
+}
+
 // NOWS: the workspace-free form (mxfa_prefill): K read as E4M3 codes and widened to bf16 in
 // LDS by p3n_widen_k at the top of every block (one K stage), V read from the caller's array;
 // VE3: V is E3M2, rewritten in LDS as E5M2 (p3n_v_e3m2_to_e5m2), O scaled by 2^12.
 // VBLK: V is E3M2 in the block-packed layout ([Skc / 32][D][24 bytes] per (b, KV head)),
 // copied into LDS as it is and read by the PV MFMA as its fp6 operand (pv_parts_blk).
-template <int D, bool SOFTCAP, int PR, bool TRACE = false, bool NOWS = false, bool VE3 = false, bool VBLK = false>
+// SPLIT (of the workspace-free form): one of a.nsplit key ranges of a query block, from the row maxima
+// of the ranges before it; leaves its partial (O, m, l) in the workspace.
+template <int D, bool SOFTCAP, int PR, bool TRACE = false, bool NOWS = false, bool VE3 = false, bool VBLK = false,
+          bool SPLIT = false>
 __device__ void prefill3_impl(const FaArgs& a) {
   using L = P3Lds<D>;
   constexpr int NW = P3Waves<D>::N;
@@ -312,11 +323,14 @@ __device__ void prefill3_impl(const FaArgs& a) {
   const int li = lin >> 3;
   const int nh_x = cnt_x / a.n_qblk;
   const bool whole_heads = start_x % a.n_qblk == 0 && cnt_x % a.n_qblk == 0;
-  const int item = start_x + (whole_heads ? (li % nh_x) * a.n_qblk + li / nh_x : li);
+  const int item = start_x + (whole_heads && !SPLIT ? (li % nh_x) * a.n_qblk + li / nh_x : li);
   const int qx = TRACE ? a.tr_qx : item % a.n_qblk, qy = TRACE ? a.tr_qy : item / a.n_qblk;
   const int qblk = a.causal ? (a.n_qblk - 1 - qx) : qx;
   const int chunks = a.group / a.hpw;
-  const int bk = qy / chunks;
+  // a split call's workgroups (a linear grid): query blocks fastest, then head chunks, key ranges
+  // and (b, KV head), so that the workgroups that read one key range are on one XCD together
+  const int ks = SPLIT ? qy / chunks % a.nsplit : 0;
+  const int bk = SPLIT ? qy / (chunks * a.nsplit) : qy / chunks;
   const int hc = qy % chunks;
   const int b = bk / a.Hkv, kvh = bk % a.Hkv;
   const int head = kvh * a.group + hc * a.hpw + (wave % a.hpw);
@@ -336,6 +350,7 @@ __device__ void prefill3_impl(const FaArgs& a) {
   int j0 = 0, j1 = nkb;
   if (a.window > 0) j0 = max(0, a.q_pos0 + q0 - a.window + 1) / BN;
   if (a.causal) j1 = min(nkb, max(0, a.q_pos0 + qmax_wg) / BN + 1);
+  if constexpr (SPLIT) split_range(a, ks, j0, j1);
   const int wq_lo = a.q_pos0 + qw0, wq_hi = a.q_pos0 + min(qw0 + 31, a.Sq - 1);
   const bool wave_live = qw0 < a.Sq;
 
@@ -364,6 +379,10 @@ __device__ void prefill3_impl(const FaArgs& a) {
 #pragma unroll
   for (int dt = 0; dt < D / 32; dt++) o[dt] = (v16f){};
   float m = -INFINITY, l = 0.0f;
+  // a later key range of a split call starts from the row maximum of the ranges before it, so its
+  // P and their codes are those of the pass over the whole range
+  if (SPLIT && qvalid)
+    for (int i = 0; i < ks; i++) m = vmax(m, a.part_max[(bh * a.Sq + qi) * a.nsplit + i]);
 
   // the wave's rows end at or past Sq (or it has none): every block is masked
   const bool edge_wave = __builtin_amdgcn_readfirstlane((qw0 + 31 >= a.Sq) || !wave_live);
@@ -479,6 +498,29 @@ __device__ void prefill3_impl(const FaArgs& a) {
   const float lt = pair_sum(l);
   // (an E3M2 V read as E5M2 carries 2^-12: undone here, exactly)
   const float inv = lt > 0.0f ? (VE3 ? 4096.0f : 1.0f) / lt : 0.0f;
+  if constexpr (SPLIT) {
+    // the range's unnormalized O, maximum and row sum, for mxfa_decode_combine (lane ids recomputed:
+    // held across the loop they spilled)
+    const float undo = VE3 ? 4096.0f : 1.0f;
+    const int ln = fresh_lane(), q = qw0 + (ln & 31);
+    const int64_t row0 = bh * a.Sq * a.nsplit + ks;
+    if (ln < 32 && q < a.Sq)
+      *reinterpret_cast<float2*>(a.part_ml + (row0 + (int64_t)q * a.nsplit) * 2) = make_float2(m, lt);
+    if constexpr (D >= 128) {
+      float* const ldsw = reinterpret_cast<float*>(
+          D == 256 ? sKb0 + wave * 8192 : (wave < 2 ? sKb0 + wave * 8192 : wave == 2 ? sV0 : sV1));
+      store_o_lds<D, false>(o, undo, ldsw, a.part_o + row0 * D, qw0, a.Sq, ln, a.nsplit * D);
+    } else if (q < a.Sq) {
+      float* orow = a.part_o + (row0 + (int64_t)q * a.nsplit) * D + 4 * (ln >> 5);
+#pragma unroll
+      for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          *reinterpret_cast<float4*>(orow + dt * 32 + 8 * g) =
+              make_float4(o[dt][4 * g] * undo, o[dt][4 * g + 1] * undo, o[dt][4 * g + 2] * undo, o[dt][4 * g + 3] * undo);
+    }
+    return;
+  }
   if constexpr (D >= 128 && !TRACE) {
     // O through LDS (store_o_lds), in a private 8 KB slice of the K tiles (one K stage at D =
     // 128: the V tiles for waves 2 and 3), free after the loop's last barrier (96 -> 68 MB
@@ -565,6 +607,137 @@ MXFA_PREFILL3N(256, false, P_R2, true, mxfa_prefill3n_d256_r2_e3m2)
 MXFA_PREFILL3N(64, true, P_R2, true, mxfa_prefill3n_d64_softcap_r2_e3m2)
 MXFA_PREFILL3N(128, true, P_R2, true, mxfa_prefill3n_d128_softcap_r2_e3m2)
 MXFA_PREFILL3N(256, true, P_R2, true, mxfa_prefill3n_d256_softcap_r2_e3m2)
+
+// Split prefill (mxfa_prefill_ws where the grid leaves the chip idle), second launch.
+#define MXFA_PREFILL3S(D, SC, PR, VE3, VBLK, NAME)                                                  \
+  extern "C" __global__ void __launch_bounds__(256, D == 256 ? 2 : 3) NAME(FaArgs a) {               \
+    prefill3_impl<D, SC, PR, false, true, VE3, VBLK, true>(a);                                       \
+  }
+#define MXFA_PREFILL3S_ALL(D)                                                                        \
+  MXFA_PREFILL3S(D, false, P_R1, false, false, mxfa_prefill3s_d##D)                                  \
+  MXFA_PREFILL3S(D, true, P_R1, false, false, mxfa_prefill3s_d##D##_softcap)                         \
+  MXFA_PREFILL3S(D, false, P_R2, false, false, mxfa_prefill3s_d##D##_r2)                             \
+  MXFA_PREFILL3S(D, true, P_R2, false, false, mxfa_prefill3s_d##D##_softcap_r2)                      \
+  MXFA_PREFILL3S(D, false, P_R1, true, false, mxfa_prefill3s_d##D##_e3m2)                            \
+  MXFA_PREFILL3S(D, true, P_R1, true, false, mxfa_prefill3s_d##D##_softcap_e3m2)                     \
+  MXFA_PREFILL3S(D, false, P_R2, true, false, mxfa_prefill3s_d##D##_r2_e3m2)                         \
+  MXFA_PREFILL3S(D, true, P_R2, true, false, mxfa_prefill3s_d##D##_softcap_r2_e3m2)                  \
+  MXFA_PREFILL3S(D, false, P_R1, false, true, mxfa_prefill3s_d##D##_blk)                             \
+  MXFA_PREFILL3S(D, true, P_R1, false, true, mxfa_prefill3s_d##D##_softcap_blk)                      \
+  MXFA_PREFILL3S(D, false, P_R2, false, true, mxfa_prefill3s_d##D##_r2_blk)                          \
+  MXFA_PREFILL3S(D, true, P_R2, false, true, mxfa_prefill3s_d##D##_softcap_r2_blk)
+MXFA_PREFILL3S_ALL(64)
+MXFA_PREFILL3S_ALL(128)
+MXFA_PREFILL3S_ALL(256)
+
+// Split prefill, first launch: the row maxima of every key range but the last (a.part_max), for
+// one query block, head chunk and range per workgroup, in the attention kernel's order (above).
+// Scores as there (p3n_widen_k, p3_qk); the capped maximum is that of the largest raw score (the
+// cap is monotone).  K alone is staged: the codes of block j + 1 land in one of two stages while
+// block j, widened from the other into the bf16 tile, is multiplied.
+template <int D, bool SOFTCAP>
+__device__ void prefill_max_impl(const FaArgs& a) {
+  using L = P3Lds<D>;
+  fp32_flush_denormals();
+  constexpr int SKS = BN * D / 32 > 256 ? BN * D / 32 : 256;
+  __shared__ __attribute__((aligned(16))) uint8_t sKb[L::KB];
+  __shared__ __attribute__((aligned(16))) uint8_t sC0[BN * D], sC1[BN * D];
+  __shared__ __attribute__((aligned(16))) uint8_t sKs0[SKS], sKs1[SKS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int nwg = (int)gridDim.x, lin = (int)blockIdx.x;
+  const int xcd = lin & 7, per = nwg >> 3, rem = nwg & 7;
+  const int item = xcd * per + min(xcd, rem) + (lin >> 3);
+  const int qx = item % a.n_qblk, qy = item / a.n_qblk;
+  const int chunks = a.group / a.hpw, nr = a.nsplit - 1;
+  const int qblk = a.causal ? (a.n_qblk - 1 - qx) : qx;
+  const int hc = qy % chunks, ks = qy / chunks % nr, bk = qy / (chunks * nr);
+  const int b = bk / a.Hkv, kvh = bk % a.Hkv;
+  const int head = kvh * a.group + hc * a.hpw + (wave % a.hpw);
+  const int q0 = qblk * a.qpw, qw0 = q0 + (wave / a.hpw) * 32, qi = qw0 + r;
+  const bool qvalid = qi < a.Sq;
+  const int64_t bh = (int64_t)b * a.Hq + head;
+  const int64_t qrow = bh * a.Sq + qi;
+  v4i qb[D / 16];
+  load_q<D>(qb, a.q + qrow * D, a.qs + qrow * (D / 32), qvalid, h);
+  const int qmax_wg = min(q0 + a.qpw, a.Sq) - 1;
+  int j0 = 0, j1 = (a.Sk + BN - 1) / BN;
+  if (a.window > 0) j0 = max(0, a.q_pos0 + q0 - a.window + 1) / BN;
+  if (a.causal) j1 = min(j1, max(0, a.q_pos0 + qmax_wg) / BN + 1);
+  split_range(a, ks, j0, j1);
+  const int wq_lo = a.q_pos0 + qw0, wq_hi = a.q_pos0 + min(qw0 + 31, a.Sq - 1);
+  int klo, khi;
+  key_limits(a, a.q_pos0 + qi, qvalid, klo, khi);
+
+  const __amdgpu_buffer_rsrc_t rk = buf_rsrc(a.k, (int64_t)bk * a.Skc * D, (int64_t)a.Sk * D);
+  const __amdgpu_buffer_rsrc_t rks = buf_rsrc(a.ks, (int64_t)bk * a.Skc * (D / 32), (int64_t)a.Sk * (D / 32));
+  const int vk = (lane % 16) * D + (lane / 16) * 16;
+  // codes of the wave's 16 rows: chunk (row lane % 16, column chunk cc) at 16 (16 cc + row)
+  auto dma = [&](uint8_t* codes, uint8_t* scales, int key0) {
+#pragma unroll
+    for (int i = 0; i < 16 * D / 1024; i++)
+      dma_lds<16>(rk, codes + wave * (16 * D) + i * 1024, vk, (key0 + 16 * wave) * D + 64 * i);
+    if (wave < (BN * D / 32 + 255) / 256) dma_lds<4>(rks, scales + wave * 256, lane * 4, key0 * (D / 32) + wave * 256);
+  };
+  float m = -INFINITY;
+  if (j0 < j1) dma(sC0, sKs0, j0 * BN);
+  auto step = [&](auto stc, int j) {
+    constexpr int ST = decltype(stc)::value;
+    const uint8_t* codes = (ST ? sC1 : sC0) + wave * (16 * D);
+    const uint8_t* scales = ST ? sKs1 : sKs0;
+    __builtin_amdgcn_s_waitcnt(0x0070 | 0x0f00 | 0);   // vmcnt(0): this wave's codes and scales have landed
+    __builtin_amdgcn_s_barrier();                      // everyone's have, and the bf16 tile is free
+    __asm__ volatile("" ::: "memory");                 // (no LDS access moves across the barriers)
+    v4i x[D / 64];
+    float f[D / 64];
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) {
+      x[i] = *reinterpret_cast<const v4i*>(codes + 16 * (lane + 64 * i));
+      f[i] = e8m0_as_float(scales[(16 * wave + lane % 16) * (D / 32) + (lane / 16 + 4 * i) / 2]);
+    }
+    if (j + 1 < j1) dma(ST ? sC0 : sC1, ST ? sKs0 : sKs1, (j + 1) * BN);
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) {
+      uint8_t* dst = sKb + wave * (32 * D) + 512 * (lane / 16 + 4 * i) + 16 * (lane % 16);
+      *reinterpret_cast<v4i*>(dst) = fp8x8_to_bf16x8((uint32_t)x[i][0], (uint32_t)x[i][1], f[i]);
+      *reinterpret_cast<v4i*>(dst + 256) = fp8x8_to_bf16x8((uint32_t)x[i][2], (uint32_t)x[i][3], f[i]);
+    }
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);                // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+    v16f s[BN / 32];
+    p3_qk<D>(s, qb, sKb, lane);
+    __asm__ volatile("" ::: "memory");
+    const int key0 = j * BN, key1 = key0 + BN - 1;
+    if (__builtin_amdgcn_readfirstlane(qw0 + 31 >= a.Sq || key1 >= a.Sk || (a.causal && key1 > wq_lo) ||
+                                       (a.window > 0 && key0 + a.window <= wq_hi)))
+      pipe_mask<false>(s, key0, klo, khi, h);
+#pragma unroll
+    for (int t = 0; t < BN / 32; t++) m = vmax(m, tile_max16(s[t]));
+  };
+  for (int j = j0; j < j1; j += 2) {
+    step(std::integral_constant<int, 0>{}, j);
+    if (j + 1 < j1) step(std::integral_constant<int, 1>{}, j + 1);
+  }
+  m = pair_max_raw(m);
+  if (SOFTCAP && !(m == -INFINITY)) {
+    const float u = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(m * (2.0f * LOG2E_F * a.sc_u)) + 1.0f);
+    m = __builtin_fmaf(-2.0f * a.cap_log2, u, a.cap_log2);
+  }
+  if (qvalid && h == 0) a.part_max[qrow * a.nsplit + ks] = m;
+}
+
+#define MXFA_PREFILL_MAX(D, SC, NAME)                                                     \
+  extern "C" __global__ void __launch_bounds__(256, D == 256 ? 2 : 4) NAME(FaArgs a) {    \
+    prefill_max_impl<D, SC>(a);                                                           \
+  }
+MXFA_PREFILL_MAX(64, false, mxfa_prefill_max_d64)
+MXFA_PREFILL_MAX(128, false, mxfa_prefill_max_d128)
+MXFA_PREFILL_MAX(256, false, mxfa_prefill_max_d256)
+MXFA_PREFILL_MAX(64, true, mxfa_prefill_max_d64_softcap)
+MXFA_PREFILL_MAX(128, true, mxfa_prefill_max_d128_softcap)
+MXFA_PREFILL_MAX(256, true, mxfa_prefill_max_d256_softcap)
 
 // Stage trace of the same kernel (one workgroup; mxfa_prefill_trace).
 #define MXFA_PREFILL3_TRACE(D, SC, PR, NAME)                                                                  \

@@ -11,8 +11,8 @@ struct FaArgs {
   const uint8_t* v;
   const uint8_t* vs;
   float* o;
-  float* part_o;      // decode: partial O  [B*Hq][nparts][D]
-  float* part_ml;     // decode: partial (m, l) [B*Hq][nparts][2]
+  float* part_o;      // decode: partial O  [B*Hq][nparts][D]; split prefill: [B*Hq*Sq][nsplit][D]
+  float* part_ml;     // decode: partial (m, l) [B*Hq][nparts][2]; split prefill: [B*Hq*Sq][nsplit][2]
   const uint8_t* kbf; // prefill: bf16 copy of K [B][Hkv][Sk][D] (mxfa_k_to_bf16)
   const uint8_t* vws; // prefill: E4M3 copy of E3M2 V [B][Hkv][Sk][D] (mxfa_k_to_bf16), else NULL
   int B, Hq, Hkv, Sq, Sk;
@@ -22,6 +22,8 @@ struct FaArgs {
   int hpw;            // prefill: query heads per workgroup
   int qpw;            // prefill: query positions per workgroup
   int n_qblk;         // prefill: query blocks; decode: interleaved partials per query head
+  int nsplit;         // prefill: key ranges per query block, each a workgroup (<= 1: the whole range)
+  float* part_max;    // split prefill: row maximum of each key range but the last [B*Hq*Sq][nsplit]
   int fuse_combine;   // decode (D <= 128): the chunks of a head merge inside the workgroup
   float c_log2;       // softmax_scale * log2(e)  (no softcap)
   float sc_u;         // softmax_scale / softcap

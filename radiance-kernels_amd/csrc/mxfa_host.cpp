@@ -65,6 +65,12 @@ const char* const kKernelNames[] = {
     "mxfa_prefill3n_d64_r2_e3m2", "mxfa_prefill3n_d128_r2_e3m2", "mxfa_prefill3n_d256_r2_e3m2",
     "mxfa_prefill3n_d64_softcap_r2_e3m2", "mxfa_prefill3n_d128_softcap_r2_e3m2", "mxfa_prefill3n_d256_softcap_r2_e3m2",
     "mxfa_quant_cols_e3m2_blk", "mxfa_kv_append_e3m2_blk",
+    "mxfa_prefill_max_d64",    "mxfa_prefill_max_d128",   "mxfa_prefill_max_d256",  "mxfa_prefill_max_d64_softcap",
+    "mxfa_prefill_max_d128_softcap", "mxfa_prefill_max_d256_softcap",
+#define MXFA_SPLIT_NAMES4(D, V) \
+  "mxfa_prefill3s_d" #D V, "mxfa_prefill3s_d" #D "_softcap" V, "mxfa_prefill3s_d" #D "_r2" V, "mxfa_prefill3s_d" #D "_softcap_r2" V
+#define MXFA_SPLIT_NAMES(D) MXFA_SPLIT_NAMES4(D, ""), MXFA_SPLIT_NAMES4(D, "_e3m2"), MXFA_SPLIT_NAMES4(D, "_blk")
+    MXFA_SPLIT_NAMES(64), MXFA_SPLIT_NAMES(128), MXFA_SPLIT_NAMES(256),
 #define MXFA_BLK_NAMES(D)                                                                                      \
   "mxfa_prefill3_d" #D "_blk", "mxfa_prefill3_d" #D "_softcap_blk", "mxfa_prefill3_d" #D "_r2_blk",            \
       "mxfa_prefill3_d" #D "_softcap_r2_blk", "mxfa_prefill3n_d" #D "_blk", "mxfa_prefill3n_d" #D "_softcap_blk", \
@@ -507,6 +513,21 @@ mxfa_status mxfa_fill_normal(float* x, int64_t n, uint64_t seed, float outlier_p
 }  // extern "C"
 
 namespace {
+// The merge of a.n_qblk partials of each of `rows` output rows (mxfa_decode_combine).
+mxfa_status launch_combine(DeviceModule* dm, FaArgs& a, int64_t rows, int D, void* stream) {
+  const int nparts = a.n_qblk;
+  void* args[] = {&a};
+  // Groups of 16 threads per workgroup of the merge: 4 up to 32 partials, where more threads
+  // cost more than their partials in flight give (24 partials of 128 heads 4.0 us against 4.1 with
+  // 16 groups and 5.0 with 64; 16 partials of 2,048 heads 6.2, 8.6 and 28), then 16 (64 partials of
+  // 128 heads 3.3 against 4.5 with 4) and above 128 partials 32 (256 of 32 heads 5.2 against
+  // 11.2 and 6.0 with 4 and 16).
+  if (nparts <= 4)
+    return launch(dm, "mxfa_decode_combine", dim3((unsigned)rows), dim3((unsigned)(D / 4)), args, stream);
+  return launch(dm, "mxfa_decode_combine", dim3((unsigned)rows, (unsigned)(D / 64)),
+                dim3(nparts <= 32 ? 64 : nparts <= 128 ? 256 : 512), args, stream);
+}
+
 // Workgroup shape of the prefill kernels: nw waves, hpw query heads (of one KV head) per
 // workgroup, nw / hpw 32-query waves each.
 FaArgs prefill_args(const mxfa_attn_params* p, const uint8_t* q, const uint8_t* q_sc, const uint8_t* k,
@@ -560,6 +581,47 @@ size_t prefill3_workspace(const mxfa_attn_params* p) {
   return prefill3_kbf_bytes(p) + v;
 }
 
+// Key ranges per query block of a mxfa_prefill_ws call (1: not split).  A few rows against a long
+// cache (a prompt chunk, drafted tokens to verify) give a grid of `items` workgroups that leaves
+// most of the chip idle for the whole walk over the keys.  Split, three launches: the row maxima
+// of every range but the last (prefill_max_impl), the attention kernel per range, starting from
+// the maximum of the ranges before it -- so every P and its code are the unsplit call's -- and
+// the merge of the partials.  O differs from the unsplit call's by the order of fp32 sums only
+// (3e-7 rel-L2 at most over 60 random calls).  Measured, unsplit -> split (ranges):
+//   Hq 32, Hkv 8, D = 128:  200 rows x 32,768 keys 1,009 -> 207 us (13), 8 x 8,192 254 -> 28 (32),
+//     8 x 1,024 36 -> 18 (11), batch 8 of 8 x 4,096 131 -> 47 (12), 512 x 16,384 391 -> 258 (3)
+//   Hq 16, Hkv 8, D = 256:  256 x 16,384 631 -> 123 (16), 30 x 2,048 softcap 111 -> 30 (16), 256 x
+//     32,768 with a window of 4,096, softcap and 6-bit V 192 -> 68 (16)
+//   Hq 16, Hkv 16, D = 64:  300 x 16,384 402 -> 75 (21)
+// - as many ranges as fill the slots the kernel's registers leave (two workgroups per CU at D =
+//   256, three at 128, four at 64), and not more than sqrt(8 x key blocks): a range's time falls
+//   with their number, the merge's grows (128 blocks: 61, 28, 30 us with 8, 32, 48 ranges; 32
+//   blocks: 24, 19, 21 with 8, 16, 24);
+// - as many partials as the workspace of the plan holds in place of the operand copies;
+// - at least 3: with 2 ranges the maxima (a third of the pass) and the merge eat the gain once
+//   there is a workgroup for most CUs (256 items: 131 against 132 us); up to 128 items 2 still win
+//   (32 x 8,192 x 8 rows 207 against 254 us);
+// - from 16 visible key blocks on (8 rows; 8 blocks: 20 -> 18 us only), and for more than one query
+//   tile per head (32 rows) in calls of more than 5,120 keys: shorter ones keep their
+//   bit-identity with mxfa_prefill, at the price of what 64 rows x 4,096 keys could gain (103 ->
+//   40 us).
+int prefill_splits(const FaArgs& a, const mxfa_attn_params* p, int64_t items) {
+  const int64_t slots = p->head_dim == 256 ? 512 : p->head_dim == 128 ? 768 : 1024;
+  const int nkb = (p->seq_k + 63) / 64;
+  int longest = 0;
+  for (int qblk = 0; qblk < a.n_qblk && slots / items > 1; qblk++) {
+    const int q0 = qblk * a.qpw, qmax = std::min(q0 + a.qpw, p->seq_q) - 1;
+    const int j0 = p->window > 0 ? std::max(0, p->q_pos0 + q0 - p->window + 1) / 64 : 0;
+    const int j1 = p->causal ? std::min(nkb, std::max(0, p->q_pos0 + qmax) / 64 + 1) : nkb;
+    longest = std::max(longest, j1 - j0);
+  }
+  if (longest < 16 || (p->seq_q > 32 && p->seq_k <= 5120)) return 1;
+  const int64_t row_bytes = (int64_t)p->batch * p->num_q_heads * p->seq_q * (p->head_dim + 3) * (int64_t)sizeof(float);
+  int64_t n = std::min(slots / items, (int64_t)std::sqrt(8.0 * longest));
+  n = std::min(n, (int64_t)prefill3_workspace(p) / row_bytes);
+  return n >= 3 || (n == 2 && items <= 128) ? (int)n : 1;
+}
+
 }  // namespace
 
 extern "C" {
@@ -611,6 +673,24 @@ mxfa_status prefill_ws_impl(const mxfa_attn_params* p, const uint8_t* q, const u
   const int nw = prefill3_waves(p);
   dim3 grid;
   FaArgs a = prefill_args(p, q, q_sc, k, k_sc, v, v_sc, o, nw, grid);
+  const int nsplit = tr ? 1 : prefill_splits(a, p, (int64_t)grid.x * grid.y);
+  if (nsplit > 1) {
+    // the workspace holds the partials instead of the operand copies: O, (m, l), row maxima
+    const int64_t rows = (int64_t)p->batch * p->num_q_heads * p->seq_q;
+    a.nsplit = nsplit;
+    a.part_o = static_cast<float*>(workspace);
+    a.part_ml = a.part_o + rows * nsplit * p->head_dim;
+    a.part_max = a.part_ml + rows * nsplit * 2;
+    const unsigned items = grid.x * grid.y;
+    void* args[] = {&a};
+    char name[64];
+    std::snprintf(name, sizeof name, "mxfa_prefill_max_d%d%s", p->head_dim, p->softcap > 0.0f ? "_softcap" : "");
+    if (mxfa_status st = launch(dm, name, dim3(items * (unsigned)(nsplit - 1)), dim3(256), args, stream)) return st;
+    if (mxfa_status st = launch(dm, kernel_name("prefill3s", p, true), dim3(items * (unsigned)nsplit), dim3(256), args, stream))
+      return st;
+    a.n_qblk = nsplit;
+    return launch_combine(dm, a, rows, p->head_dim, stream);
+  }
   if (!tr && prefill_ws_widens_in_lds(a, p)) {
     void* args[] = {&a};
     return launch(dm, kernel_name("prefill3n", p, true), grid, dim3(256), args, stream);
@@ -711,15 +791,7 @@ mxfa_status decode_launch(DeviceModule* dm, const mxfa_attn_params* p, const uin
                               stream))
     return st;
   if (a.fuse_combine) return MXFA_OK;
-  // Groups of 16 threads per workgroup of the merge: 4 up to 32 partials, where more threads
-  // cost more than their partials in flight give (24 partials of 128 heads 4.0 us against 4.1 with
-  // 16 groups and 5.0 with 64; 16 partials of 2,048 heads 6.2, 8.6 and 28), then 16 (64 partials of
-  // 128 heads 3.3 against 4.5 with 4) and above 128 partials 32 (256 of 32 heads 5.2 against
-  // 11.2 and 6.0 with 4 and 16).
-  if (nparts <= 4)
-    return launch(dm, "mxfa_decode_combine", dim3((unsigned)nbh), dim3((unsigned)(p->head_dim / 4)), args, stream);
-  return launch(dm, "mxfa_decode_combine", dim3((unsigned)nbh, (unsigned)(p->head_dim / 64)),
-                dim3(nparts <= 32 ? 64 : nparts <= 128 ? 256 : 512), args, stream);
+  return launch_combine(dm, a, nbh, p->head_dim, stream);
 }
 
 }  // namespace

@@ -45,3 +45,39 @@ def test_decode_merge_part_counts(monkeypatch, parts):
     rel, mab = errors(np_(o), want)
     print(f"   n_parts {n_parts}: rel-L2 {rel:.3e} max-abs {mab:.3e}", flush=True)
     assert rel <= REL_L2_TOL and mab <= MAX_ABS_TOL
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,n,D,kw", [
+    (1, 8, 2, 1, 1024, 128, {}),                                        # 16 key blocks: the shortest split range
+    (1, 8, 2, 32, 2000, 128, dict(v_fmt=mxfa.FMT_E3M2)),                # a full query tile, last block partly filled
+    (2, 14, 2, 31, 1100, 64, dict(v_fmt=mxfa.FMT_E3M2_BLK, p_rule=mxfa.P_R2)),
+    (1, 4, 2, 5, 3001, 256, dict(softcap=30.0, window=1500)),           # ranges that start inside the window
+    (1, 2, 1, 33, 5200, 256, dict(v_fmt=mxfa.FMT_E3M2, softcap=30.0)),  # two query tiles, 82 key blocks
+    (1, 16, 4, 100, 5152, 128, {}),                                     # two tiles: the shortest such call
+    (1, 8, 4, 40, 6000, 256, dict(window=1200, v_fmt=mxfa.FMT_E3M2_BLK)),
+    (1, 3, 3, 64, 5300, 64, dict(causal=False)),
+    (1, 4, 1, 17, 4096, 128, dict(short=2200)),                         # queries far before the end: ranges past them empty
+])
+def test_split_prefill_matches_single_pass(B, Hq, Hkv, Sq, n, D, kw):
+    """mxfa_prefill_ws split over the keys against mxfa_prefill (one pass): the same P codes, so O
+    differs by fp32 summation order alone.  Each of the at most 32 partials is rounded once more
+    when it is scaled and added: 32 x 2^-24 = 2e-6 of the row."""
+    Sk = (n + 31) // 32 * 32
+    v_fmt = kw.get("v_fmt", mxfa.FMT_E4M3)
+    causal = kw.get("causal", True)
+    pos0 = kw.get("short", n - Sq) if causal else 0
+    _, dev, host = gen_qkv(B, Hq, Hkv, Sq, Sk, D, seed=300 + n, outlier_p=0.01, v_fmt=v_fmt)
+    p = mxfa.make_params(B, Hq, Hkv, Sq, Sk, D, causal=causal, q_pos0=pos0, window=kw.get("window", 0),
+                         softcap=kw.get("softcap", 0.0), v_fmt=v_fmt, p_rule=kw.get("p_rule", mxfa.P_R1))
+    ops = [dev[x] for x in ("q", "qs", "k", "ks", "v", "vs")]
+    out = torch.full((B, Hq, Sq, D), float("nan"), dtype=torch.float32, device=DEV)
+    ws = torch.full((mxfa.prefill_plan(p),), 255, dtype=torch.uint8, device=DEV)      # NaN wherever a partial is read unwritten
+    mxfa.prefill(p, *ops, out=out, workspace=ws)
+    one = mxfa.prefill(p, *ops, workspace=False)
+    again = mxfa.prefill(p, *ops, workspace=ws)
+    torch.cuda.synchronize()
+    assert not torch.equal(out, one), "the call was not split"
+    assert torch.equal(out, again)
+    rel, _ = errors(np_(out), np_(one))
+    print(f"   split against one pass: rel-L2 {rel:.3e}", flush=True)
+    assert rel <= 2e-6
