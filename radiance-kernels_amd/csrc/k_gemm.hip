@@ -565,6 +565,365 @@ extern "C" __global__ void __launch_bounds__(64 * MXFA_GEMM_DMA_WAVES, 1) mxfa_g
 }
 
 // ---------------------------------------------------------------------------
+// Mid-size MX GEMM: 128 x 128 tiles, for shapes whose 256 x 256 tiles leave CUs idle (M = 400, N = 6,144:
+// 48 of them on 256 CUs).  Four waves of 64 x 64 (2 x 2 MFMA tiles), one per SIMD, so each wave
+// interleaves its own work: a step's operands are read from LDS in four parts, one behind each MFMA
+// of the half step before, and the staging of later steps behind the MFMAs too.  The LDS tiles are
+// unpadded, their 16-byte chunks XOR-swizzled: A row r chunk c at c ^ ((r >> 1) & 7), B k row k
+// chunk c at c ^ 2 ((k >> 1) & 3) (a ds_read_b64_tr_b8 takes two chunks of eight k rows: rows k and
+// k + 1 are the two halves of the 64 banks).  Every accumulator adds the same products in the same
+// order as in the 256 x 256 kernels.  Measured (M = 400, N = 6,144, K = 4,096, E4M3, bf16 C): 256 x
+// 256 42.8 us, this tile register-staged 25.5, with the reads ahead of the MFMAs 24.9, LDS DMA 18.4,
+// reads between the MFMAs 16.0 (0.32 us per step of 512 MFMA clocks; 8 MB of A and B per us).
+//
+// Register-staged form, for E3M2 operands (widened to E4M3 on the way into LDS): the operands of
+// step kt + R are loaded R steps ahead with plain loads, whose waits stay partial, and stored to the
+// other of two LDS stages; two workgroups per CU.  Everything at k >= K, rows >= M and columns >=
+// N reads as zero.
+// ---------------------------------------------------------------------------
+namespace gmid {
+constexpr int T = 128, TK = 128, KB = TK / 32;
+constexpr int A_BYTES = T * TK, S_BYTES = 2 * KB * T;   // A and B alike; SA [KB][T] then SB [KB][T]
+constexpr int STAGE = 2 * A_BYTES + S_BYTES;
+constexpr int R = 2;
+}  // namespace gmid
+
+struct GmidStage {
+  v4i a[4], b[4];
+  uint32_t s;
+};
+
+struct GmidSrc {
+  __amdgpu_buffer_rsrc_t a, b, s;
+  uint32_t va[4], vb[4], vs;               // vector offsets of the thread's chunks at k = 0
+  int acol;                                // k of its A chunks within a step
+  int K, N, sdim;
+};
+
+__device__ __forceinline__ void gmid_load(GmidStage& st, const GmidSrc& src, int k0) {
+  const uint32_t dis = (uint32_t)(src.acol + k0 >= src.K) << 31;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    st.a[i] = __builtin_amdgcn_raw_buffer_load_b128(src.a, src.va[i] | dis, k0, 0);
+    st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(src.b, src.vb[i], k0 * src.N, 0);
+  }
+  st.s = __builtin_amdgcn_raw_buffer_load_b32(src.s, src.vs, (k0 / 32) * src.sdim, 0);
+}
+
+// Part i of 4 of a step's LDS stores (the scales with part 0).
+template <int AE3, int BE3>
+__device__ __forceinline__ void gmid_store(const GmidStage& st, uint8_t* stage, int tid, int i) {
+  using namespace gmid;
+  {
+    const int c = tid + 256 * i, row = c >> 3, ch = c & 7;
+    v4i va = st.a[i], vb = st.b[i];
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      if (AE3) va[w] = (int)e3m2x4_to_e4m3x4((uint32_t)va[w]);
+      if (BE3) vb[w] = (int)e3m2x4_to_e4m3x4((uint32_t)vb[w]);
+    }
+    *reinterpret_cast<v4i*>(stage + row * TK + ((ch ^ ((row >> 1) & 7)) << 4)) = va;
+    *reinterpret_cast<v4i*>(stage + A_BYTES + row * T + ((ch ^ (2 * ((row >> 1) & 3))) << 4)) = vb;
+  }
+  if (i == 0) *reinterpret_cast<uint32_t*>(stage + 2 * A_BYTES + 4 * tid) = st.s;
+}
+
+// The wave's operands of one 64-k half of a step.
+struct GmidOps {
+  v8i a[2], b[2];
+  int as[2], bs[2];
+};
+
+// Part p of 4 of their reads (B and A of tile p / 2): one part behind each MFMA of the half before.
+__device__ __forceinline__ void gmid_read(GmidOps& o, const uint8_t* stage, int kh, int wr, int wc, int lane, int p) {
+  using namespace gmid;
+  const int r = lane & 31, h = lane >> 5, l16 = lane & 15, g16 = lane >> 4;
+  const uint8_t* sB = stage + A_BYTES;
+  const uint8_t* sS = stage + 2 * A_BYTES;
+  const int u = p >> 1;
+  if (p % 2 == 0) {
+    const int ncol = 64 * wc + 32 * u + 16 * (g16 & 1) + 8 * (l16 & 1);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int krow = 64 * kh + 32 * (q >> 1) + 16 * h + 8 * (q & 1) + (l16 >> 1);
+      const int addr = krow * T + (((ncol >> 4) ^ (2 * ((krow >> 1) & 3))) << 4) + (ncol & 15);
+      const v2i t = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(sB + addr));
+      o.b[u][2 * q] = t[0];
+      o.b[u][2 * q + 1] = t[1];
+    }
+    o.bs[u] = sS[KB * T + (2 * kh + h) * T + 64 * wc + 32 * u + r];
+  } else {
+    const int row = 64 * wr + 32 * u + r, sw = (row >> 1) & 7;
+    o.a[u] = cat44(*reinterpret_cast<const v4i*>(stage + row * TK + (((4 * kh + h) ^ sw) << 4)),
+                   *reinterpret_cast<const v4i*>(stage + row * TK + (((4 * kh + 2 + h) ^ sw) << 4)));
+    o.as[u] = sS[(2 * kh + h) * T + row];
+  }
+}
+
+__device__ __forceinline__ void gmid_mma(v16f (&acc)[2][2], const GmidOps& o, int i) {
+  acc[i >> 1][i & 1] = mfma_mx(o.a[i >> 1], o.b[i & 1], acc[i >> 1][i & 1], o.as[i >> 1], o.bs[i & 1]);
+}
+
+// XCD-aware grouped tile order as the 256 x 256 kernels, in groups of 8 tile rows.
+__device__ __forceinline__ void gmid_tile(const GemmArgs& g, int& m0, int& n0) {
+  using namespace gmid;
+  constexpr int GM = 8;
+  const int nwg = (int)gridDim.x, lin = (int)blockIdx.x;
+  const int xcd = lin & 7, per = nwg >> 3, rem = nwg & 7;
+  const int item = xcd * per + min(xcd, rem) + (lin >> 3);
+  const int tiles_m = (g.M + T - 1) / T;
+  const int group = item / (GM * g.tiles_n), first = group * GM, gm = min(GM, tiles_m - first);
+  const int in_group = item - group * GM * g.tiles_n;
+  m0 = (first + in_group % gm) * T;
+  n0 = (in_group / gm) * T;
+}
+
+// C through LDS, as the 256 x 256 DMA kernel: each wave stages its 64 x 64 tile in its 16 KB of lds and
+// stores whole lines.
+__device__ __forceinline__ void gmid_store_c(const GemmArgs& g, const v16f (&acc)[2][2], uint8_t* lds, int m0, int n0,
+                                             int wave, int lane) {
+  using namespace gmid;
+  const int r = lane & 31, h = lane >> 5, wr = wave >> 1, wc = wave & 1;
+  uint8_t* const reg = lds + wave * (64 * 64 * 4);
+  auto epilogue = [&](auto es_c) {
+    constexpr int ES = decltype(es_c)::value;
+    constexpr int W = 64 * ES, RPI = 1024 / W;
+    const int rows = min(T, g.M - m0);
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(g.c + (int64_t)m0 * g.N * ES), 0, (int)(uint32_t)((int64_t)rows * g.N * ES), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          uint8_t* const e = reg + (32 * i + 8 * (v >> 2) + 4 * h + (v & 3)) * W + (32 * j + r) * ES;
+          if constexpr (ES == 4) *reinterpret_cast<float*>(e) = acc[i][j][v];
+          else *reinterpret_cast<__bf16*>(e) = (__bf16)acc[i][j][v];
+        }
+#pragma unroll
+    for (int u = 0; u < 64 / RPI; u++) {
+      const int lr = u * RPI + lane / (W / 16), ch = lane % (W / 16);
+      const v4i x = *reinterpret_cast<const v4i*>(reg + lr * W + ch * 16);
+      const int col = n0 + 64 * wc + ch * (16 / ES);
+      const uint32_t off = col < g.N ? (uint32_t)((64 * wr + lr) * g.N + col) * (uint32_t)ES : 0xfffffff0u;
+      __builtin_amdgcn_raw_buffer_store_b128(x, rc, off, 0, 0);
+    }
+  };
+  if (g.c_bf16)
+    epilogue(std::integral_constant<int, 2>{});
+  else
+    epilogue(std::integral_constant<int, 4>{});
+}
+
+template <int AE3, int BE3>
+__device__ __forceinline__ void gemm_mid_impl(const GemmArgs& g) {
+  using namespace gmid;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int m0, n0;
+  gmid_tile(g, m0, n0);
+  const int wr = wave >> 1, wc = wave & 1;
+
+  GmidSrc src;
+  src.K = g.K;
+  src.N = g.N;
+  src.a = buf_rsrc(g.a, (int64_t)m0 * g.K, (int64_t)(g.M - m0) * g.K);
+  src.b = buf_rsrc(g.b, 0, (int64_t)g.K * g.N);
+  src.acol = 16 * (tid & 7);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int row = (tid >> 3) + 32 * i, bc = n0 + 16 * (tid & 7);
+    src.va[i] = (uint32_t)(row * g.K + src.acol);
+    src.vb[i] = bc < g.N ? (uint32_t)(row * g.N + bc) : 0x80000000u;
+  }
+  {
+    const bool is_a = wave < 2;                      // wave-uniform: the scale resource stays scalar
+    const int t = tid & 127, c = (is_a ? m0 : n0) + 4 * (t & 31);
+    src.sdim = is_a ? g.M : g.N;
+    src.s = buf_rsrc(is_a ? g.sa : g.sb, 0, (int64_t)(g.K / 32) * src.sdim);
+    src.vs = c < src.sdim ? (uint32_t)((t >> 5) * src.sdim + c) : 0x80000000u;
+  }
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (v16f){};
+
+  const int nk = (g.K + TK - 1) / TK;
+  GmidStage st[R];
+#pragma unroll
+  for (int u = 0; u < R; u++) gmid_load(st[u], src, u * TK);
+#pragma unroll
+  for (int i = 0; i < 4; i++) gmid_store<AE3, BE3>(st[0], lds, tid, i);
+  __syncthreads();
+  GmidOps o0, o1;
+#pragma unroll
+  for (int i = 0; i < 4; i++) gmid_read(o0, lds, 0, wr, wc, lane, i);
+  // Step kt from stage kt % 2, its first half's operands already in registers: the second half's are
+  // read and step kt + 1 is stored (from slot (kt + 1) % R) between the first half's MFMAs; after
+  // the barrier the next step's first operands are read between the second half's.  Slot kt % R,
+  // stored a step ago, takes step kt + R (past the last step: zeros, never multiplied).
+  auto step = [&](auto uc, int kt) {
+    constexpr int u = decltype(uc)::value;
+    const uint8_t* cur = lds + (u & 1) * STAGE;
+    uint8_t* nxt = lds + ((u + 1) & 1) * STAGE;
+    gmid_load(st[u % R], src, (kt + R) * TK);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      gmid_mma(acc, o0, i);
+      __builtin_amdgcn_sched_barrier(0);
+      gmid_read(o1, cur, 1, wr, wc, lane, i);
+      gmid_store<AE3, BE3>(st[(u + 1) % R], nxt, tid, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      gmid_mma(acc, o1, i);
+      __builtin_amdgcn_sched_barrier(0);
+      gmid_read(o0, nxt, 0, wr, wc, lane, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr int U = 2 * R / (R % 2 ? 1 : 2);          // slots and stages repeat every U steps
+  for (int kt = 0; kt < nk; kt += U) {
+    step(std::integral_constant<int, 0>{}, kt);
+    if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
+    if constexpr (U > 2) {
+      if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
+      if (kt + 3 < nk) step(std::integral_constant<int, 3>{}, kt + 3);
+      if (kt + 4 < nk) step(std::integral_constant<int, 4>{}, kt + 4);
+      if (kt + 5 < nk) step(std::integral_constant<int, 5>{}, kt + 5);
+    }
+  }
+  __syncthreads();
+
+  gmid_store_c(g, acc, lds, m0, n0, wave, lane);
+}
+
+// The same tile for E4M3 operands, staged by LDS DMA through four stages, the DMA of step kt + 4
+// issued in step kt: one wave per SIMD has nothing to cover the LDS stores and register loads of
+// the form above with (0.63 us per step; 0.31 without both).  The DMA instructions are inline
+// assembly without outputs: the compiler would make every LDS read wait for every DMA in flight
+// (vmcnt(0)); here the waits are explicit, for the one stage read next.  Per step each wave issues
+// 4 A, 4 B and one scale instruction (GMID_DMA), always, also past the last step (zeros or rows
+// that are never multiplied), so that vmcnt counts whole stages.
+constexpr int GMID_DMA = 9, GMID_S = 4;
+
+__device__ __forceinline__ v4i rsrc_words(const uint8_t* base, int64_t off, int64_t bytes) {
+  const uint64_t p = (uint64_t)(uintptr_t)(base + off);
+  return (v4i){(int)(uint32_t)p, (int)(uint32_t)((p >> 32) & 0xffffu), (int)(bytes > 0 ? bytes : 0), 0x00020000};
+}
+__device__ __forceinline__ void dma_asm16(v4i rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void dma_asm4(v4i rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+
+__device__ __forceinline__ void gemm_mid_dma_impl(const GemmArgs& g) {
+  using namespace gmid;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[GMID_S * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int m0, n0;
+  gmid_tile(g, m0, n0);
+  const int wr = wave >> 1, wc = wave & 1;
+
+  const v4i ra = rsrc_words(g.a, (int64_t)m0 * g.K, (int64_t)(g.M - m0) * g.K);
+  const v4i rb = rsrc_words(g.b, 0, (int64_t)g.K * g.N);
+  const bool is_a = wave < 2;
+  const int sdim = is_a ? g.M : g.N;
+  const v4i rs = rsrc_words(is_a ? g.sa : g.sb, 0, (int64_t)(g.K / 32) * sdim);
+  // instruction i: A rows or B k rows 8 i .. 8 i + 7, lane l row l / 8, LDS chunk l % 8
+  uint32_t va[2], vb, vs;
+#pragma unroll
+  for (int par = 0; par < 2; par++)
+    va[par] = (uint32_t)((lane / 8) * g.K + 16 * ((lane % 8) ^ (((8 * par + lane / 8) >> 1) & 7)));
+  {
+    const int bc = n0 + 16 * ((lane % 8) ^ (2 * ((lane >> 4) & 3)));
+    vb = bc < g.N ? (uint32_t)((lane / 8) * g.N + bc) : 0x80000000u;
+    const int c = (is_a ? m0 : n0) + 4 * (lane & 31);
+    vs = c < sdim ? (uint32_t)((lane >> 5) * sdim + c) : 0x80000000u;
+  }
+  const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_addr(lds));
+  // part q of 4 of the DMA of step kt into stage `slot` (the scales with part 0)
+  auto dma = [&](int slot, int kt, int q) {
+    const uint32_t st = base + (uint32_t)slot * STAGE;
+    const int k0 = kt * TK, i = 4 * wave + q;
+    dma_asm16(ra, st + i * 1024, va[q & 1], (uint32_t)(8 * i * g.K + k0));
+    dma_asm16(rb, st + A_BYTES + i * 1024, vb, (uint32_t)(k0 + 8 * i) * (uint32_t)g.N);
+    if (q == 0) dma_asm4(rs, st + 2 * A_BYTES + wave * 256, vs, (uint32_t)(k0 / 32 + 2 * (wave & 1)) * (uint32_t)sdim);
+  };
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (v16f){};
+#pragma unroll
+  for (int u = 0; u < GMID_S; u++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) dma(u, u, q);
+  __asm__ volatile("s_waitcnt vmcnt(%0)" : : "i"(3 * GMID_DMA) : "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+  GmidOps o0, o1;
+#pragma unroll
+  for (int i = 0; i < 4; i++) gmid_read(o0, lds, 0, wr, wc, lane, i);
+  const int nk = g.K / TK;                             // whole steps; K % 128 == 64 leaves a half one
+  auto step = [&](auto uc, int kt) {
+    constexpr int u = decltype(uc)::value;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      gmid_mma(acc, o0, i);
+      __builtin_amdgcn_sched_barrier(0);
+      gmid_read(o1, lds + u * STAGE, 1, wr, wc, lane, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // stage kt + 1 has landed (two later ones in flight) and, after the barrier, everyone's has;
+    // stage kt is read out and takes step kt + 4
+    __asm__ volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "i"(2 * GMID_DMA) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      gmid_mma(acc, o1, i);
+      __builtin_amdgcn_sched_barrier(0);
+      gmid_read(o0, lds + (u + 1) % GMID_S * STAGE, 0, wr, wc, lane, i);
+      dma(u, kt + GMID_S, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int kt = 0; kt < nk; kt += GMID_S) {
+    step(std::integral_constant<int, 0>{}, kt);
+    if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
+    if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
+    if (kt + 3 < nk) step(std::integral_constant<int, 3>{}, kt + 3);
+  }
+  if (g.K % TK) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) gmid_mma(acc, o0, i);
+  }
+  // every DMA has landed before the stages are reused
+  __asm__ volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  __syncthreads();
+  gmid_store_c(g, acc, lds, m0, n0, wave, lane);
+}
+
+extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_mid_dma(GemmArgs g) { gemm_mid_dma_impl(g); }
+
+#define MXFA_GEMM_MID(AE, BE, NAME) \
+  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs g) { gemm_mid_impl<AE, BE>(g); }
+MXFA_GEMM_MID(1, 0, mxfa_gemm_mid_ae3m2)
+MXFA_GEMM_MID(0, 1, mxfa_gemm_mid_be3m2)
+MXFA_GEMM_MID(1, 1, mxfa_gemm_mid_ae3m2_be3m2)
+
+// ---------------------------------------------------------------------------
 // Skinny MX GEMM (M <= 32 T rows, E4M3 x E4M3): the batched-decode projection, where the big
 // kernel's 256 x 256 tiles leave the chip idle (N / 256 workgroups) and the weights B stream
 // at a few percent of HBM.  One workgroup per 32-column strip of B and C (strips contiguous

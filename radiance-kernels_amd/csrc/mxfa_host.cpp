@@ -65,6 +65,7 @@ const char* const kKernelNames[] = {
     "mxfa_prefill3n_d64_r2_e3m2", "mxfa_prefill3n_d128_r2_e3m2", "mxfa_prefill3n_d256_r2_e3m2",
     "mxfa_prefill3n_d64_softcap_r2_e3m2", "mxfa_prefill3n_d128_softcap_r2_e3m2", "mxfa_prefill3n_d256_softcap_r2_e3m2",
     "mxfa_quant_cols_e3m2_blk", "mxfa_kv_append_e3m2_blk",
+    "mxfa_gemm_mid_dma", "mxfa_gemm_mid_ae3m2", "mxfa_gemm_mid_be3m2", "mxfa_gemm_mid_ae3m2_be3m2",
     "mxfa_prefill_max_d64",    "mxfa_prefill_max_d128",   "mxfa_prefill_max_d256",  "mxfa_prefill_max_d64_softcap",
     "mxfa_prefill_max_d128_softcap", "mxfa_prefill_max_d256_softcap",
 #define MXFA_SPLIT_NAMES4(D, V) \
@@ -475,20 +476,43 @@ mxfa_status mxfa_gemm(const mxfa_gemm_params* p, const uint8_t* a, const uint8_t
                                           {"mxfa_gemm_ae3m2", "mxfa_gemm_ae3m2_be3m2"}};
   const int64_t tm = (p->m + 255) / 256, tn = (p->n + 255) / 256;
   g.tiles_n = (int)tn;
-  // the kernels are built for one workgroup size (their launch bounds): 256 or 512 threads.
-  // E4M3 operands with whole K steps (k % 128 == 0) take the LDS-DMA kernel
-  // (MXFA_GEMM=reg selects the register-staged one, for comparison).
+  // MXFA_GEMM selects a kernel for comparison: big or dma the 256 x 256 tiles (big also below M =
+  // 128), reg their register-staged form, mid the 128 x 128 tiles
   const char* sel = getenv("MXFA_GEMM");
-  // M <= 128 with E4M3 operands (the batched-decode projection): the skinny kernel, one
-  // workgroup per 32-column strip (MXFA_GEMM=big or =reg selects the tiled kernels instead)
-  // (its LDS holds all of SA and the strip's SB: (k / 32) (m + 32) <= 96 KiB)
-  if (!g.a_e3m2 && !g.b_e3m2 && p->m <= 128 && (p->k / 32) * (p->m + 32) <= 96 * 1024 &&
-      !(sel && (std::strcmp(sel, "big") == 0 || std::strcmp(sel, "reg") == 0))) {
+  auto selected = [&](const char* name) { return sel && std::strcmp(sel, name) == 0; };
+  const bool e4m3 = !g.a_e3m2 && !g.b_e3m2;
+  // M <= 128 with E4M3 operands (the batched-decode projection): the skinny kernel, one workgroup per
+  // 32-column strip (its LDS holds all of SA and the strip's SB: (k / 32) (m + 32) <= 96 KiB), while
+  // the strips fit the chip at once (N = 14,336: 28 against 18 us for the 128 x 128 tiles at M = 64,
+  // 37 against 20 at 128; N = 6,144: 15 against 16 at M = 64), and above M = 64 only for K > 4,096
+  // (N = 4,096, M = 128: 16.4 against 15.2 us at K = 4,096, 48.5 against 52.7 at 14,336).
+  const int64_t strips = (p->n + 31) / 32;
+  if (e4m3 && p->m <= 128 && (p->k / 32) * (p->m + 32) <= 96 * 1024 && strips <= 256 && (p->m <= 64 || p->k > 4096) &&
+      !selected("big") && !selected("reg") && !selected("mid")) {
     const char* sk = p->m <= 32 ? "mxfa_gemm_skinny_t1" : p->m <= 64 ? "mxfa_gemm_skinny_t2" : "mxfa_gemm_skinny_t4";
     void* args[] = {&g};
-    return launch(dm, sk, dim3((unsigned)((p->n + 31) / 32)), dim3(256), args, stream);
+    return launch(dm, sk, dim3((unsigned)strips), dim3(256), args, stream);
   }
-  const bool dma = !g.a_e3m2 && !g.b_e3m2 && p->k % 128 == 0 && !(sel && std::strcmp(sel, "reg") == 0);
+  // 128 x 128 tiles (the same sums in the same order) while the 256 x 256 tiles are at most two
+  // rounds over the CUs and the smaller ones at most twice as many: a K step of 128 takes 0.32 us
+  // against 1.1.  N = 6,144, K = 4,096: M = 400 16 against 43 us, 1,024 (384 tiles of 128) 36 against
+  // 44; 2,048 (768, three rounds against one) 57 against 47.  With E3M2 operands (two workgroups
+  // per CU): M = 400 35 against 69 us, 1,024 50 against 69.
+  const int64_t tiles128 = (p->m + 127) / 128 * ((p->n + 127) / 128);
+  const int64_t rounds256 = (tm * tn + 255) / 256;
+  if (selected("mid") || (!sel && rounds256 <= 2 &&
+                          (e4m3 ? (tiles128 + 255) / 256 <= 2 * rounds256 : (tiles128 + 511) / 512 <= rounds256))) {
+    g.tiles_n = (int)((p->n + 127) / 128);
+    const char* mid = e4m3         ? "mxfa_gemm_mid_dma"
+                      : !g.a_e3m2  ? "mxfa_gemm_mid_be3m2"
+                      : !g.b_e3m2  ? "mxfa_gemm_mid_ae3m2"
+                                   : "mxfa_gemm_mid_ae3m2_be3m2";
+    void* args[] = {&g};
+    return launch(dm, mid, dim3((unsigned)tiles128), dim3(256), args, stream);
+  }
+  // The 256 x 256 kernels are built for one workgroup size (their launch bounds): 256 or 512
+  // threads.  E4M3 operands with whole K steps (k % 128 == 0) take the LDS-DMA kernel.
+  const bool dma = e4m3 && p->k % 128 == 0 && !selected("reg");
   const char* name = dma ? "mxfa_gemm_dma" : names[g.a_e3m2][g.b_e3m2];
   int threads = 0;
   MXFA_HIP(hipFuncGetAttribute(&threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, fn_by_name(dm, name)));

@@ -81,3 +81,38 @@ def test_split_prefill_matches_single_pass(B, Hq, Hkv, Sq, n, D, kw):
     rel, _ = errors(np_(out), np_(one))
     print(f"   split against one pass: rel-L2 {rel:.3e}", flush=True)
     assert rel <= 2e-6
+
+
+@pytest.mark.parametrize("M,N,K,a_fmt,b_fmt", [
+    (144, 128, 64, 0, 0),            # one half step only
+    (160, 80, 192, 0, 0),            # a step and a half, columns and rows past the tile
+    (128, 8208, 128, 0, 0),          # one step: three of the four stages hold nothing; more strips than CUs
+    (400, 1040, 576, 0, 0),          # 4 whole steps and a half, ragged
+    (1024, 4096, 640, 0, 0),         # 256 tiles
+    (272, 272, 1088, 0, 1), (256, 144, 64, 1, 0), (48, 400, 320, 1, 1),
+])
+def test_gemm_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_fmt, b_fmt):
+    """The 128 x 128 tiles run the MFMAs of the 256 x 256 kernels on the same operands in the same
+    order: C must match bit for bit, fp32 and bf16, NaN codes past the edges of A and B unread."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M + N + K)
+
+    def codes(fmt, shape):
+        c = torch.randint(0, 256 if fmt == 0 else 64, shape, generator=g, device=DEV, dtype=torch.int32)
+        return torch.where((c & 127) == 127, c - 1, c).to(torch.uint8)
+
+    a, b = codes(a_fmt, (M, K)), codes(b_fmt, (K, N))
+    sa, sb = (torch.randint(112, 142, (K // 32, n), generator=g, device=DEV, dtype=torch.int32).to(torch.uint8) for n in (M, N))
+    for c_fmt, dt in ((mxfa.C_F32, torch.float32), (mxfa.C_BF16, torch.bfloat16)):
+        outs = []
+        for mode in (None, "reg"):
+            if mode:
+                monkeypatch.setenv("MXFA_GEMM", mode)
+            else:
+                monkeypatch.delenv("MXFA_GEMM", raising=False)
+            c = torch.full((M, N), float("nan"), dtype=dt, device=DEV)
+            mxfa.gemm(a, sa, b, sb, a_fmt, b_fmt, out=c, c_fmt=c_fmt)
+            outs.append(c)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(outs[0]).all())
+        assert torch.equal(outs[0], outs[1])
