@@ -267,32 +267,49 @@ const char* kernel_name(const char* kind, const mxfa_attn_params* p, bool v_suff
 }
 
 // Split-KV plan: the 64-key blocks of each (b, KV head) are dealt to n_parts interleaved
-// partials (partial i: blocks i, i + n_parts, ...), one wave each, about kDecodeWaves
-// partial waves per call -- two per SIMD of the 256-CU chip, at the two workgroups per CU
-// of D <= 128; half as many at D = 256, whose kernel fits one workgroup per CU (measured
-// on B32 Hq16 Hkv8 L8192 D256: 0.169 ms at 1,024 waves, 0.182 at 2,048).  At most 4 partials are
-// rounded up to 1, 2 or 4 so that a head's partials fill whole 4-wave workgroups and merge
-// inside them.  Interleaving puts the partial waves of a head, which share a workgroup,
-// on adjacent blocks at the same time (measured on c5: 188 us vs 204 us for contiguous
-// chunks at 2048 waves).  MXFA_DECODE_WAVES overrides the target.
+// partials (partial i: blocks i, i + n_parts, ...), one wave each, four to a workgroup.
+// Interleaving puts the partial waves of a head, which share a workgroup, on adjacent blocks at
+// the same time (measured on c5: 188 us vs 204 us for contiguous chunks at 2048 waves).
+//
+// At most about kDecodeWaves partial waves per call -- two per SIMD of the 256-CU chip, at the two
+// workgroups per CU of D <= 128; half as many at D = 256, whose kernel fits one workgroup per CU
+// (measured on B32 Hq16 Hkv8 L8192 D256: 0.169 ms at 1,024 waves, 0.182 at 2,048).  At most 4
+// partials are rounded up to 1, 2 or 4 so that a head's partials fill whole 4-wave workgroups and
+// merge inside them.  The workspace is sized for this many; MXFA_DECODE_WAVES overrides the target
+// and then exactly so many are used.
 constexpr int64_t kDecodeWaves = 2048;
 
-int64_t decode_wave_target(int head_dim) {
-  if (const char* env = getenv("MXFA_DECODE_WAVES")) {
-    long long v = atoll(env);
-    if (v > 0) return v;
-  }
-  return head_dim == 256 ? kDecodeWaves / 2 : kDecodeWaves;
+int64_t decode_wave_override() {
+  const char* env = getenv("MXFA_DECODE_WAVES");
+  const long long v = env ? atoll(env) : 0;
+  return v > 0 ? v : 0;
 }
 
-int decode_parts(const mxfa_attn_params* p) {
+int decode_parts_max(const mxfa_attn_params* p) {
   const int64_t bk = (int64_t)p->batch * p->num_kv_heads;
   const int64_t blocks = (p->seq_k + 63) / 64;
-  int64_t n = (decode_wave_target(p->head_dim) + bk - 1) / bk;
+  int64_t target = decode_wave_override();
+  if (target == 0) target = p->head_dim == 256 ? kDecodeWaves / 2 : kDecodeWaves;
+  int64_t n = (target + bk - 1) / bk;
   if (n == 3) n = 4;
   if (n > blocks) n = blocks;
   if (n < 1) n = 1;
   return (int)n;
+}
+
+// Of those, no more than the blocks that the query sees: with a window in a longer cache the other
+// partials are empty (window 4,096 in a cache of 60,000 keys: 65 of 938 blocks visible, 256 partials
+// 14.1 us a call, 65 12.6).  Each visible block is then a partial of its own in either plan, so O
+// differs by the order of the merge's fp32 sums only.  (Fewer partials than that can be faster
+// -- 96 heads of 47 blocks at D = 256, 264 workgroups on 256 CUs in 11 partials each: 50.2 us, in 10
+// 32.7 -- but change the running maxima that P is quantized against.)
+int decode_parts(const mxfa_attn_params* p) {
+  const int nmax = decode_parts_max(p);
+  if (p->window <= 0 || decode_wave_override()) return nmax;
+  const int hi = p->causal ? std::min(p->seq_k - 1, p->q_pos0) : p->seq_k - 1;
+  const int lo = std::max(0, p->q_pos0 - p->window + 1);
+  const int vis = hi >= lo ? hi / 64 - lo / 64 + 1 : 1;
+  return std::min(nmax, vis == 3 ? 4 : vis);
 }
 
 }  // namespace
@@ -776,10 +793,11 @@ mxfa_status mxfa_prefill_trace(const mxfa_attn_params* p, const uint8_t* q, cons
 
 mxfa_status mxfa_decode_plan(const mxfa_attn_params* p, int32_t* n_parts, size_t* workspace_bytes) {
   if (mxfa_status st = check_params(p, true)) return st;
-  const int np = decode_parts(p);
-  if (n_parts) *n_parts = np;
+  if (n_parts) *n_parts = decode_parts(p);
+  // sized for the most partials a call of this shape could take, so that it never shrinks with a
+  // longer cache
   if (workspace_bytes)
-    *workspace_bytes = (size_t)p->batch * p->num_q_heads * np * (p->head_dim + 2) * sizeof(float) + 256;
+    *workspace_bytes = (size_t)p->batch * p->num_q_heads * decode_parts_max(p) * (p->head_dim + 2) * sizeof(float) + 256;
   return MXFA_OK;
 }
 
