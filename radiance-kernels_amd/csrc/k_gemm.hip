@@ -665,36 +665,36 @@ __device__ __forceinline__ void gmid_mma(v16f (&acc)[2][2], const GmidOps& o, in
 }
 
 // XCD-aware grouped tile order as the 256 x 256 kernels, in groups of 8 tile rows.
+template <int TM, int TN>
 __device__ __forceinline__ void gmid_tile(const GemmArgs& g, int& m0, int& n0) {
-  using namespace gmid;
   constexpr int GM = 8;
   const int nwg = (int)gridDim.x, lin = (int)blockIdx.x;
   const int xcd = lin & 7, per = nwg >> 3, rem = nwg & 7;
   const int item = xcd * per + min(xcd, rem) + (lin >> 3);
-  const int tiles_m = (g.M + T - 1) / T;
+  const int tiles_m = (g.M + TM - 1) / TM;
   const int group = item / (GM * g.tiles_n), first = group * GM, gm = min(GM, tiles_m - first);
   const int in_group = item - group * GM * g.tiles_n;
-  m0 = (first + in_group % gm) * T;
-  n0 = (in_group / gm) * T;
+  m0 = (first + in_group % gm) * TM;
+  n0 = (in_group / gm) * TN;
 }
 
-// C through LDS, as the 256 x 256 DMA kernel: each wave stages its 64 x 64 tile in its 16 KB of lds and
-// stores whole lines.
-__device__ __forceinline__ void gmid_store_c(const GemmArgs& g, const v16f (&acc)[2][2], uint8_t* lds, int m0, int n0,
+// C through LDS, as the 256 x 256 DMA kernel: each wave stages its 32 TI x 32 TJ tile in its own part
+// of lds and stores whole lines.
+template <int TI, int TJ>
+__device__ __forceinline__ void gmid_store_c(const GemmArgs& g, const v16f (&acc)[TI][TJ], uint8_t* lds, int m0, int n0,
                                              int wave, int lane) {
-  using namespace gmid;
   const int r = lane & 31, h = lane >> 5, wr = wave >> 1, wc = wave & 1;
-  uint8_t* const reg = lds + wave * (64 * 64 * 4);
+  uint8_t* const reg = lds + wave * (32 * TI * 32 * TJ * 4);
   auto epilogue = [&](auto es_c) {
     constexpr int ES = decltype(es_c)::value;
-    constexpr int W = 64 * ES, RPI = 1024 / W;
-    const int rows = min(T, g.M - m0);
+    constexpr int W = 32 * TJ * ES, RPI = 1024 / W;
+    const int rows = min(64 * TI, g.M - m0);
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(g.c + (int64_t)m0 * g.N * ES), 0, (int)(uint32_t)((int64_t)rows * g.N * ES), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < TI; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < TJ; j++)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
           uint8_t* const e = reg + (32 * i + 8 * (v >> 2) + 4 * h + (v & 3)) * W + (32 * j + r) * ES;
@@ -702,11 +702,11 @@ __device__ __forceinline__ void gmid_store_c(const GemmArgs& g, const v16f (&acc
           else *reinterpret_cast<__bf16*>(e) = (__bf16)acc[i][j][v];
         }
 #pragma unroll
-    for (int u = 0; u < 64 / RPI; u++) {
+    for (int u = 0; u < 32 * TI / RPI; u++) {
       const int lr = u * RPI + lane / (W / 16), ch = lane % (W / 16);
       const v4i x = *reinterpret_cast<const v4i*>(reg + lr * W + ch * 16);
-      const int col = n0 + 64 * wc + ch * (16 / ES);
-      const uint32_t off = col < g.N ? (uint32_t)((64 * wr + lr) * g.N + col) * (uint32_t)ES : 0xfffffff0u;
+      const int col = n0 + 32 * TJ * wc + ch * (16 / ES);
+      const uint32_t off = col < g.N ? (uint32_t)((32 * TI * wr + lr) * g.N + col) * (uint32_t)ES : 0xfffffff0u;
       __builtin_amdgcn_raw_buffer_store_b128(x, rc, off, 0, 0);
     }
   };
@@ -722,7 +722,7 @@ __device__ __forceinline__ void gemm_mid_impl(const GemmArgs& g) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int m0, n0;
-  gmid_tile(g, m0, n0);
+  gmid_tile<gmid::T, gmid::T>(g, m0, n0);
   const int wr = wave >> 1, wc = wave & 1;
 
   GmidSrc src;
@@ -801,17 +801,22 @@ __device__ __forceinline__ void gemm_mid_impl(const GemmArgs& g) {
   }
   __syncthreads();
 
-  gmid_store_c(g, acc, lds, m0, n0, wave, lane);
+  gmid_store_c<2, 2>(g, acc, lds, m0, n0, wave, lane);
 }
 
-// The same tile for E4M3 operands, staged by LDS DMA through four stages, the DMA of step kt + 4
-// issued in step kt: one wave per SIMD has nothing to cover the LDS stores and register loads of
-// the form above with (0.63 us per step; 0.31 without both).  The DMA instructions are inline
-// assembly without outputs: the compiler would make every LDS read wait for every DMA in flight
-// (vmcnt(0)); here the waits are explicit, for the one stage read next.  Per step each wave issues
-// 4 A, 4 B and one scale instruction (GMID_DMA), always, also past the last step (zeros or rows
-// that are never multiplied), so that vmcnt counts whole stages.
-constexpr int GMID_DMA = 9, GMID_S = 4;
+// E4M3 operands, staged by LDS DMA: tiles of 64 TI x 64 TJ, four waves (2 x 2) of TI x TJ MFMA tiles,
+// one per SIMD, 128 NSUB k per stage, GDMA_S stages, the DMA of stage t + 4 issued in stage t.  One
+// wave per SIMD has nothing to cover the LDS stores and register loads of the form above with (128 x
+// 128: 0.63 us per 128 k; 0.31 without both).  The DMA instructions are inline assembly without
+// outputs: the compiler would make every LDS read wait for every DMA in flight (vmcnt(0)); here the
+// waits are explicit, for the one stage read next.  Every wave issues the same number of DMA
+// instructions per stage, always, also past the last one (zeros or rows that are never
+// multiplied), so that vmcnt counts whole stages.  A stage's operands are read into registers during
+// the stage before, each behind the MFMA that last used its register.
+// 128 x 128 (mid, one sub-stage of 128 k) and, where even those leave CUs idle, 64 x 64 (small, two
+// sub-stages: one barrier per 256 k, as a wave has one MFMA per 64 k): M = 128, N = 4,096, K = 4,096
+// 13.5 and 8.3 us (operands in L2), N = 6,144 18.3 and 13.3 (25 MB of weights from the MALL).
+constexpr int GDMA_S = 4;
 
 __device__ __forceinline__ v4i rsrc_words(const uint8_t* base, int64_t off, int64_t bytes) {
   const uint64_t p = (uint64_t)(uintptr_t)(base + off);
@@ -826,96 +831,177 @@ __device__ __forceinline__ void dma_asm4(v4i rsrc, uint32_t lds, uint32_t voff, 
                    : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
 }
 
-__device__ __forceinline__ void gemm_mid_dma_impl(const GemmArgs& g) {
-  using namespace gmid;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[GMID_S * STAGE];
+template <int TI, int TJ, int NSUB> struct GdmaCfg {
+  static constexpr int TM = 64 * TI, TN = 64 * TJ, TK = 128;         // TK: one sub-stage
+  static constexpr int A_BYTES = TM * TK, B_BYTES = TN * TK, SA = 4 * TM, SB = 4 * TN;
+  static constexpr int SUB = A_BYTES + B_BYTES + SA + SB, STAGE = NSUB * SUB;
+  static constexpr int AI = A_BYTES / 4096, BI = B_BYTES / 4096;     // instructions per wave and sub-stage
+  static constexpr int DMA = NSUB * (AI + BI + 1);                   // per wave and stage
+  static_assert(3 * DMA <= 63, "vmcnt range");
+};
+
+// The wave's operands of one 64-k half of a sub-stage; the B chunk swizzle as A's, by what part of the
+// 64 banks a k row of 64 TJ bytes covers.
+template <int TI, int TJ> struct GdmaOps {
+  v8i a[TI], b[TJ];
+  int as[TI], bs[TJ];
+};
+template <int TJ> __device__ __forceinline__ int gdma_swb(int krow) {
+  return TJ == 2 ? 2 * ((krow >> 1) & 3) : 2 * ((krow >> 2) & 1);
+}
+
+// Part p of TI * TJ of a half's reads.
+template <int TI, int TJ, int NSUB>
+__device__ __forceinline__ void gdma_read(GdmaOps<TI, TJ>& o, const uint8_t* sub, int kh, int wr, int wc, int lane, int p) {
+  using C = GdmaCfg<TI, TJ, NSUB>;
+  const int r = lane & 31, h = lane >> 5, l16 = lane & 15, g16 = lane >> 4;
+  const uint8_t *sB = sub + C::A_BYTES, *sSA = sB + C::B_BYTES, *sSB = sSA + C::SA;
+#pragma unroll
+  for (int j = 0; j < TJ; j++) {
+    if (j != p * TJ / (TI * TJ) || p * TJ % (TI * TJ) != 0) continue;
+    const int ncol = 32 * TJ * wc + 32 * j + 16 * (g16 & 1) + 8 * (l16 & 1);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int krow = 64 * kh + 32 * (q >> 1) + 16 * h + 8 * (q & 1) + (l16 >> 1);
+      const int addr = krow * C::TN + (((ncol >> 4) ^ gdma_swb<TJ>(krow)) << 4) + (ncol & 15);
+      const v2i t = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(sB + addr));
+      o.b[j][2 * q] = t[0];
+      o.b[j][2 * q + 1] = t[1];
+    }
+    o.bs[j] = sSB[(2 * kh + h) * C::TN + 32 * TJ * wc + 32 * j + r];
+  }
+#pragma unroll
+  for (int i = 0; i < TI; i++) {
+    if ((TI * TJ == 1 ? 0 : 2 * i + 1) != p) continue;
+    const int row = 32 * TI * wr + 32 * i + r, sw = (row >> 1) & 7;
+    o.a[i] = cat44(*reinterpret_cast<const v4i*>(sub + row * 128 + (((4 * kh + h) ^ sw) << 4)),
+                   *reinterpret_cast<const v4i*>(sub + row * 128 + (((4 * kh + 2 + h) ^ sw) << 4)));
+    o.as[i] = sSA[(2 * kh + h) * C::TM + row];
+  }
+}
+
+template <int TI, int TJ, int NSUB>
+__device__ __forceinline__ void gemm_dma_tile_impl(const GemmArgs& g) {
+  using C = GdmaCfg<TI, TJ, NSUB>;
+  constexpr int NP = TI * TJ, HALVES = 2 * NSUB;
+  static_assert(TI == TJ && (TI == 1 || TI == 2), "tile shapes");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[GDMA_S * C::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int m0, n0;
-  gmid_tile(g, m0, n0);
+  gmid_tile<C::TM, C::TN>(g, m0, n0);
   const int wr = wave >> 1, wc = wave & 1;
 
   const v4i ra = rsrc_words(g.a, (int64_t)m0 * g.K, (int64_t)(g.M - m0) * g.K);
   const v4i rb = rsrc_words(g.b, 0, (int64_t)g.K * g.N);
-  const bool is_a = wave < 2;
+  const bool is_a = TI == 2 ? wave < 2 : (wave & 1) == 0;
   const int sdim = is_a ? g.M : g.N;
   const v4i rs = rsrc_words(is_a ? g.sa : g.sb, 0, (int64_t)(g.K / 32) * sdim);
-  // instruction i: A rows or B k rows 8 i .. 8 i + 7, lane l row l / 8, LDS chunk l % 8
+  // A instruction i: rows 8 i .. 8 i + 7, lane l row l / 8, LDS chunk l % 8; B instruction i: BR k rows of
+  // 64 TJ bytes.  Scales: 256 bytes per instruction, 4 / TI k groups of the 64 TI columns (64 x
+  // 64 tiles: SA and SB whole, by two waves each, the same bytes twice).
+  constexpr int BR = 16 / TJ, BC = 4 * TJ;
   uint32_t va[2], vb, vs;
 #pragma unroll
   for (int par = 0; par < 2; par++)
     va[par] = (uint32_t)((lane / 8) * g.K + 16 * ((lane % 8) ^ (((8 * par + lane / 8) >> 1) & 7)));
   {
-    const int bc = n0 + 16 * ((lane % 8) ^ (2 * ((lane >> 4) & 3)));
-    vb = bc < g.N ? (uint32_t)((lane / 8) * g.N + bc) : 0x80000000u;
-    const int c = (is_a ? m0 : n0) + 4 * (lane & 31);
-    vs = c < sdim ? (uint32_t)((lane >> 5) * sdim + c) : 0x80000000u;
+    const int bc = n0 + 16 * ((lane % BC) ^ gdma_swb<TJ>(lane / BC));
+    vb = bc < g.N ? (uint32_t)((lane / BC) * g.N + bc) : 0x80000000u;
+    const int c = (is_a ? m0 : n0) + 4 * (lane % (16 * TI));
+    vs = c < sdim ? (uint32_t)((lane / (16 * TI)) * sdim + c) : 0x80000000u;
   }
+  const int skb = TI == 2 ? 2 * (wave & 1) : 0;        // first k group of the wave's scale instruction
+  const uint32_t sdst = C::A_BYTES + C::B_BYTES + (is_a ? 0 : C::SA) + skb * C::TM;
   const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_addr(lds));
-  // part q of 4 of the DMA of step kt into stage `slot` (the scales with part 0)
-  auto dma = [&](int slot, int kt, int q) {
-    const uint32_t st = base + (uint32_t)slot * STAGE;
-    const int k0 = kt * TK, i = 4 * wave + q;
-    dma_asm16(ra, st + i * 1024, va[q & 1], (uint32_t)(8 * i * g.K + k0));
-    dma_asm16(rb, st + A_BYTES + i * 1024, vb, (uint32_t)(k0 + 8 * i) * (uint32_t)g.N);
-    if (q == 0) dma_asm4(rs, st + 2 * A_BYTES + wave * 256, vs, (uint32_t)(k0 / 32 + 2 * (wave & 1)) * (uint32_t)sdim);
+  // part q of PARTS of the DMA of stage t into `slot` (a sub-stage's scales with its first part)
+  static_assert(C::AI == C::BI, "square tiles");
+  constexpr int PARTS = NSUB * C::AI;
+  auto dma = [&](int slot, int t, int q) {
+    const int sub = q / C::AI, i = C::AI * wave + q % C::AI;
+    const uint32_t st = base + (uint32_t)(slot * C::STAGE + sub * C::SUB);
+    const int k0 = (t * NSUB + sub) * C::TK;
+    dma_asm16(ra, st + i * 1024, va[i & 1], (uint32_t)(8 * i * g.K + k0));
+    dma_asm16(rb, st + C::A_BYTES + i * 1024, vb, (uint32_t)(k0 + BR * i) * (uint32_t)g.N);
+    if (q % C::AI == 0) dma_asm4(rs, st + sdst, vs, (uint32_t)(k0 / 32 + skb) * (uint32_t)sdim);
   };
 
-  v16f acc[2][2];
+  v16f acc[TI][TJ];
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < TI; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = (v16f){};
+    for (int j = 0; j < TJ; j++) acc[i][j] = (v16f){};
+  GdmaOps<TI, TJ> o[HALVES];                           // one set per half of a stage
+  auto mma = [&](int s, int i) {
+    acc[i / TJ][i % TJ] = mfma_mx(o[s].a[i / TJ], o[s].b[i % TJ], acc[i / TJ][i % TJ], o[s].as[i / TJ], o[s].bs[i % TJ]);
+  };
+  auto read = [&](int s, int slot, int hh, int p) {
+    gdma_read<TI, TJ, NSUB>(o[s], lds + slot * C::STAGE + (hh >> 1) * C::SUB, hh & 1, wr, wc, lane, p);
+  };
+
 #pragma unroll
-  for (int u = 0; u < GMID_S; u++)
+  for (int u = 0; u < GDMA_S; u++)
 #pragma unroll
-    for (int q = 0; q < 4; q++) dma(u, u, q);
-  __asm__ volatile("s_waitcnt vmcnt(%0)" : : "i"(3 * GMID_DMA) : "memory");
+    for (int q = 0; q < PARTS; q++) dma(u, u, q);
+  __asm__ volatile("s_waitcnt vmcnt(%0)" : : "i"(3 * C::DMA) : "memory");
   __builtin_amdgcn_s_barrier();
   __asm__ volatile("" ::: "memory");
-  GmidOps o0, o1;
 #pragma unroll
-  for (int i = 0; i < 4; i++) gmid_read(o0, lds, 0, wr, wc, lane, i);
-  const int nk = g.K / TK;                             // whole steps; K % 128 == 64 leaves a half one
-  auto step = [&](auto uc, int kt) {
+  for (int hh = 0; hh < HALVES; hh++)
+#pragma unroll
+    for (int p = 0; p < NP; p++) read(hh, 0, hh, p);
+  const int nh = g.K / 64;                             // halves in all
+  // Stage t, its operands in registers: once stage t + 1 has landed (two later ones in flight) and, at
+  // the barrier, everyone's has and stage t is read out, the MFMAs, and behind each a part of the
+  // same half's reads of stage t + 1 and of the DMA of stage t + 4.
+  auto stage = [&](auto uc, int t) {
     constexpr int u = decltype(uc)::value;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      gmid_mma(acc, o0, i);
-      __builtin_amdgcn_sched_barrier(0);
-      gmid_read(o1, lds + u * STAGE, 1, wr, wc, lane, i);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // stage kt + 1 has landed (two later ones in flight) and, after the barrier, everyone's has;
-    // stage kt is read out and takes step kt + 4
-    __asm__ volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "i"(2 * GMID_DMA) : "memory");
+    __asm__ volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "i"(2 * C::DMA) : "memory");
     __builtin_amdgcn_s_barrier();
     __asm__ volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      gmid_mma(acc, o1, i);
+    for (int k = 0; k < HALVES * NP; k++) {
+      mma(k / NP, k % NP);
       __builtin_amdgcn_sched_barrier(0);
-      gmid_read(o0, lds + (u + 1) % GMID_S * STAGE, 0, wr, wc, lane, i);
-      dma(u, kt + GMID_S, i);
+      // (2 x 2 tiles in the order 00, 01, 10, 11 free A0 after 01, B0 after 10, B1 and A1 after 11;
+      // A1 is read behind the next half's first MFMA)
+      if constexpr (NP == 1) {
+        read(k, (u + 1) % GDMA_S, k, 0);
+      } else {
+        if (k % 4 == 1) read(k / 4, (u + 1) % GDMA_S, k / 4, 1);
+        if (k % 4 == 2) read(k / 4, (u + 1) % GDMA_S, k / 4, 0);
+        if (k % 4 == 3) read(k / 4, (u + 1) % GDMA_S, k / 4, 2);
+        if (k % 4 == 3 && k / 4 == HALVES - 1) read(k / 4, (u + 1) % GDMA_S, k / 4, 3);
+        if (k % 4 == 0 && k / 4 > 0) read(k / 4 - 1, (u + 1) % GDMA_S, k / 4 - 1, 3);
+      }
+#pragma unroll
+      for (int q = k * PARTS / (HALVES * NP); q < (k + 1) * PARTS / (HALVES * NP); q++) dma(u, t + GDMA_S, q);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  for (int kt = 0; kt < nk; kt += GMID_S) {
-    step(std::integral_constant<int, 0>{}, kt);
-    if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
-    if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
-    if (kt + 3 < nk) step(std::integral_constant<int, 3>{}, kt + 3);
+  const int nst = nh / HALVES;
+  int t = 0;
+  for (; t + GDMA_S <= nst; t += GDMA_S) {
+    stage(std::integral_constant<int, 0>{}, t);
+    stage(std::integral_constant<int, 1>{}, t + 1);
+    stage(std::integral_constant<int, 2>{}, t + 2);
+    stage(std::integral_constant<int, 3>{}, t + 3);
   }
-  if (g.K % TK) {
+  if (t < nst) stage(std::integral_constant<int, 0>{}, t);
+  if (t + 1 < nst) stage(std::integral_constant<int, 1>{}, t + 1);
+  if (t + 2 < nst) stage(std::integral_constant<int, 2>{}, t + 2);
+  // the halves of a last stage that is not whole
+  const int left = nh - nst * HALVES;
 #pragma unroll
-    for (int i = 0; i < 4; i++) gmid_mma(acc, o0, i);
-  }
+  for (int k = 0; k < (HALVES - 1) * NP; k++)
+    if (k / NP < left) mma(k / NP, k % NP);
   // every DMA has landed before the stages are reused
   __asm__ volatile("s_waitcnt vmcnt(0)" : : : "memory");
   __syncthreads();
-  gmid_store_c(g, acc, lds, m0, n0, wave, lane);
+  gmid_store_c<TI, TJ>(g, acc, lds, m0, n0, wave, lane);
 }
 
-extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_mid_dma(GemmArgs g) { gemm_mid_dma_impl(g); }
+extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_mid_dma(GemmArgs g) { gemm_dma_tile_impl<2, 2, 1>(g); }
+extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_small_dma(GemmArgs g) { gemm_dma_tile_impl<1, 1, 2>(g); }
 
 #define MXFA_GEMM_MID(AE, BE, NAME) \
   extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs g) { gemm_mid_impl<AE, BE>(g); }
@@ -924,7 +1010,7 @@ MXFA_GEMM_MID(0, 1, mxfa_gemm_mid_be3m2)
 MXFA_GEMM_MID(1, 1, mxfa_gemm_mid_ae3m2_be3m2)
 
 // ---------------------------------------------------------------------------
-// Skinny MX GEMM (M <= 32 T rows, E4M3 x E4M3): the batched-decode projection, where the big
+// Skinny MX GEMM (M <= 32 T rows, T = 1 or 2, E4M3 x E4M3): the batched-decode projection, where the big
 // kernel's 256 x 256 tiles leave the chip idle (N / 256 workgroups) and the weights B stream
 // at a few percent of HBM.  One workgroup per 32-column strip of B and C (strips contiguous
 // per XCD, so the four strips that share each 128-byte line of a B row share one L2).  The
@@ -944,10 +1030,10 @@ MXFA_GEMM_MID(1, 1, mxfa_gemm_mid_ae3m2_be3m2)
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_SCALE_BYTES = 96 * 1024;                   // (K / 32) (M + 32) at most
 
-// Ring slots (steps in flight per wave).  Measured on M = 16 / 64 / 128 (N 6144, K 4096): 8 / 6 /
-// 4 slots 11.3 / 17.0 / 25.7 us, the vmcnt limit (16 / 11 / 7) 14.1 / 18.2 / 26.4 us.
+// Ring slots (steps in flight per wave).  Measured on M = 16 / 64 (N 6144, K 4096): 8 / 6 slots
+// 11.3 / 17.0 us, the vmcnt limit (16 / 11) 14.1 / 18.2 us.
 template <int T> struct SkinnyCfg {
-  static constexpr int R = T == 1 ? 8 : T == 2 ? 6 : 4;
+  static constexpr int R = T == 1 ? 8 : 6;
   static constexpr int AP = 80;                                  // A row pitch in the slab (bytes)
   static constexpr int SLAB = 2048 + T * 32 * AP;                // per-wave slab: B [64][32], A tiles
   static_assert(4 * SLAB >= 4 * 16 * 64 * 4, "the partials reuse the slabs");
@@ -1148,7 +1234,6 @@ __device__ void gemm_skinny_impl(const GemmArgs& g) {
 
 extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_skinny_t1(GemmArgs g) { gemm_skinny_impl<1>(g); }
 extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_skinny_t2(GemmArgs g) { gemm_skinny_impl<2>(g); }
-extern "C" __global__ void __launch_bounds__(256, 1) mxfa_gemm_skinny_t4(GemmArgs g) { gemm_skinny_impl<4>(g); }
 
 // Waves per GEMM workgroup; the host reads the workgroup size from the kernel's
 // launch bounds (its maximum threads per block).

@@ -55,7 +55,7 @@ const char* const kKernelNames[] = {
     "mxfa_prefill3_trace_d64_softcap", "mxfa_prefill3_trace_d128_softcap", "mxfa_prefill3_trace_d256_softcap",
     "mxfa_prefill3_trace_d64_r2", "mxfa_prefill3_trace_d128_r2", "mxfa_prefill3_trace_d256_r2",
     "mxfa_prefill3_trace_d64_softcap_r2", "mxfa_prefill3_trace_d128_softcap_r2", "mxfa_prefill3_trace_d256_softcap_r2",
-    "mxfa_gemm_dma", "mxfa_gemm_skinny_t1", "mxfa_gemm_skinny_t2", "mxfa_gemm_skinny_t4",
+    "mxfa_gemm_dma", "mxfa_gemm_skinny_t1", "mxfa_gemm_skinny_t2",
     "mxfa_prefill3n_d64", "mxfa_prefill3n_d128", "mxfa_prefill3n_d256", "mxfa_prefill3n_d64_softcap",
     "mxfa_prefill3n_d128_softcap", "mxfa_prefill3n_d256_softcap", "mxfa_prefill3n_d64_r2", "mxfa_prefill3n_d128_r2",
     "mxfa_prefill3n_d256_r2", "mxfa_prefill3n_d64_softcap_r2", "mxfa_prefill3n_d128_softcap_r2",
@@ -65,7 +65,7 @@ const char* const kKernelNames[] = {
     "mxfa_prefill3n_d64_r2_e3m2", "mxfa_prefill3n_d128_r2_e3m2", "mxfa_prefill3n_d256_r2_e3m2",
     "mxfa_prefill3n_d64_softcap_r2_e3m2", "mxfa_prefill3n_d128_softcap_r2_e3m2", "mxfa_prefill3n_d256_softcap_r2_e3m2",
     "mxfa_quant_cols_e3m2_blk", "mxfa_kv_append_e3m2_blk",
-    "mxfa_gemm_mid_dma", "mxfa_gemm_mid_ae3m2", "mxfa_gemm_mid_be3m2", "mxfa_gemm_mid_ae3m2_be3m2",
+    "mxfa_gemm_mid_dma", "mxfa_gemm_small_dma", "mxfa_gemm_mid_ae3m2", "mxfa_gemm_mid_be3m2", "mxfa_gemm_mid_ae3m2_be3m2",
     "mxfa_prefill_max_d64",    "mxfa_prefill_max_d128",   "mxfa_prefill_max_d256",  "mxfa_prefill_max_d64_softcap",
     "mxfa_prefill_max_d128_softcap", "mxfa_prefill_max_d256_softcap",
 #define MXFA_SPLIT_NAMES4(D, V) \
@@ -498,20 +498,30 @@ mxfa_status mxfa_gemm(const mxfa_gemm_params* p, const uint8_t* a, const uint8_t
   const char* sel = getenv("MXFA_GEMM");
   auto selected = [&](const char* name) { return sel && std::strcmp(sel, name) == 0; };
   const bool e4m3 = !g.a_e3m2 && !g.b_e3m2;
-  // M <= 128 with E4M3 operands (the batched-decode projection): the skinny kernel, one workgroup per
+  // M <= 64 with E4M3 operands (the batched-decode projection): the skinny kernel, one workgroup per
   // 32-column strip (its LDS holds all of SA and the strip's SB: (k / 32) (m + 32) <= 96 KiB), while
-  // the strips fit the chip at once (N = 14,336: 28 against 18 us for the 128 x 128 tiles at M = 64,
-  // 37 against 20 at 128; N = 6,144: 15 against 16 at M = 64), and above M = 64 only for K > 4,096
-  // (N = 4,096, M = 128: 16.4 against 15.2 us at K = 4,096, 48.5 against 52.7 at 14,336).
+  // the strips fit the chip at once (N = 14,336, M = 64: 28 us, the tiles below 16) and, above M =
+  // 32, only for a long K (us at K = 4,096, N = 6,144, skinny and 64 x 64 tiles: M = 16 11.4 and 12.2,
+  // 32 12.4 and 12.5, 64 14.8 and 13.4; K = 14,336, N = 4,096: 30.6 and 35.1, 32.0 and 36.4, 38.9 and
+  // 40.7; K = 7,168, N = 2,048, M = 64 13.2 and 10.6).
   const int64_t strips = (p->n + 31) / 32;
-  if (e4m3 && p->m <= 128 && (p->k / 32) * (p->m + 32) <= 96 * 1024 && strips <= 256 && (p->m <= 64 || p->k > 4096) &&
+  if (e4m3 && p->m <= 64 && (p->k / 32) * (p->m + 32) <= 96 * 1024 && strips <= 256 && (p->m <= 32 || p->k > 8192) &&
       !selected("big") && !selected("reg") && !selected("mid")) {
-    const char* sk = p->m <= 32 ? "mxfa_gemm_skinny_t1" : p->m <= 64 ? "mxfa_gemm_skinny_t2" : "mxfa_gemm_skinny_t4";
     void* args[] = {&g};
-    return launch(dm, sk, dim3((unsigned)strips), dim3(256), args, stream);
+    return launch(dm, p->m <= 32 ? "mxfa_gemm_skinny_t1" : "mxfa_gemm_skinny_t2", dim3((unsigned)strips), dim3(256), args,
+                  stream);
+  }
+  // 64 x 64 tiles while there is a CU for each (E4M3; us for 64 and 128 tiles at K = 4,096: M = 128, N =
+  // 6,144 13.3 and 18.3, M = 256, N = 4,096 9.9 and 13.6, M = N = 1,024 10.2 and 17.1; more than one
+  // round, M = 400, N = 4,096: 20.4 and 14.0)
+  const int64_t tiles64 = (p->m + 63) / 64 * ((p->n + 63) / 64);
+  if (!sel && e4m3 && tiles64 <= 256) {
+    g.tiles_n = (int)((p->n + 63) / 64);
+    void* args[] = {&g};
+    return launch(dm, "mxfa_gemm_small_dma", dim3((unsigned)tiles64), dim3(256), args, stream);
   }
   // 128 x 128 tiles (the same sums in the same order) while the 256 x 256 tiles are at most two
-  // rounds over the CUs and the smaller ones at most twice as many: a K step of 128 takes 0.32 us
+  // rounds over the CUs and the smaller ones at most twice as many: a K step of 128 takes 0.3 us
   // against 1.1.  N = 6,144, K = 4,096: M = 400 16 against 43 us, 1,024 (384 tiles of 128) 36 against
   // 44; 2,048 (768, three rounds against one) 57 against 47.  With E3M2 operands (two workgroups
   // per CU): M = 400 35 against 69 us, 1,024 50 against 69.

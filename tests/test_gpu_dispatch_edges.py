@@ -84,16 +84,22 @@ def test_split_prefill_matches_single_pass(B, Hq, Hkv, Sq, n, D, kw):
 
 
 @pytest.mark.parametrize("M,N,K,a_fmt,b_fmt", [
-    (144, 128, 64, 0, 0),            # one half step only
-    (160, 80, 192, 0, 0),            # a step and a half, columns and rows past the tile
-    (128, 8208, 128, 0, 0),          # one step: three of the four stages hold nothing; more strips than CUs
-    (400, 1040, 576, 0, 0),          # 4 whole steps and a half, ragged
+    # 64 x 64 tiles (256 k per stage)
+    (48, 64, 64, 0, 0),              # one half: no whole stage
+    (80, 144, 192, 0, 0),            # three halves, rows and columns past the tile
+    (128, 8192, 256, 0, 0),          # one stage, 256 tiles; three of the four stages hold nothing
+    (1024, 1024, 1344, 0, 0),        # 5 whole stages and a half
+    (16, 8208, 512, 0, 0),           # more strips than CUs
+    # 128 x 128 tiles
+    (144, 6208, 64, 0, 0),           # one half step only
+    (160, 6160, 192, 0, 0),          # a step and a half, columns and rows past the tile
+    (400, 4112, 576, 0, 0),          # 4 whole steps and a half, ragged
     (1024, 4096, 640, 0, 0),         # 256 tiles
     (272, 272, 1088, 0, 1), (256, 144, 64, 1, 0), (48, 400, 320, 1, 1),
 ])
-def test_gemm_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_fmt, b_fmt):
-    """The 128 x 128 tiles run the MFMAs of the 256 x 256 kernels on the same operands in the same
-    order: C must match bit for bit, fp32 and bf16, NaN codes past the edges of A and B unread."""
+def test_gemm_small_and_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_fmt, b_fmt):
+    """The 64 x 64 and 128 x 128 tiles run the MFMAs of the 256 x 256 kernels on the same operands in
+    the same order: C must match bit for bit, fp32 and bf16."""
     g = torch.Generator(device=DEV)
     g.manual_seed(M + N + K)
 
