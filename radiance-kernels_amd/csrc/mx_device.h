@@ -7,38 +7,28 @@
 //                  bits, saturating at 448           (lib/golden/mx_fp_math.h:205-225)
 //   E3M2 element : bf16 RNE, then RNE to E4M2, then the fixed E4M2 -> E3M2 value
 //                  map                                (lib/golden/mx_fp_math.h:11-28, 266-335)
-// floorf(log2f(x)) is reproduced from the exponent plus a per-binade mantissa
-// threshold (log2f rounds to float, so values just below 2^(e+1) give e+1).
+// floorf(log2f(x)) is reproduced from the exponent plus a mantissa threshold (log2f rounds to
+// float, so values just below 2^(e+1) give e+1).
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "e3m2_rule.h"
-#include "log2_table.h"
 
 namespace mxfa {
 
-__constant__ uint32_t c_log2_thr[256] = MXFA_LOG2_THR_INIT;
-__constant__ uint32_t c_log2_sub_thr[23] = MXFA_LOG2_SUB_THR_INIT;
-
-// floorf(log2f(x)) for finite x > 0 (x == 0 returns a large negative number).
-__device__ __forceinline__ int floor_log2f(float x) {
-  uint32_t b = __float_as_uint(x) & 0x7fffffffu;
-  uint32_t E = b >> 23, m = b & 0x7fffffu;
-  if (E == 0) {
-    if (m == 0) return -1024;
-    int p = 31 - __clz(m);
-    return p - 149 + (m >= c_log2_sub_thr[p] ? 1 : 0);
-  }
-  return (int)E - 127 + (m >= c_log2_thr[E] ? 1 : 0);
-}
-
-// E8M0 block scale code; amax = max |x| over the block (NaN already dropped by fmaxf).
+// E8M0 block scale code; amax = max |x| over the block (NaN already dropped by fmaxf).  floorf(log2f())
+// as in scale_code_p below (a table of the thresholds per exponent, as here before, gives the same
+// code for every one of the 2^31 floats, log2_pmax 8 and 4, and costs a dependent load per block).
+// Zero, infinite and NaN amax give 0.
 __device__ __forceinline__ uint32_t scale_code(float amax, int log2_pmax) {
-  if (!(amax > 0.0f) || __builtin_isinf(amax)) return 0u;
-  int s2 = floor_log2f(amax) - log2_pmax + 127;
-  return (uint32_t)(s2 < 0 ? 0 : (s2 > 254 ? 254 : s2));
+  const uint32_t b = __float_as_uint(amax);
+  const int e = (int)(b >> 23) - 127;
+  const uint32_t u = (uint32_t)(e ^ (e >> 31));      // e >= 0 ? e : -e - 1
+  const uint32_t delta = (uint32_t)((0x2C160B05020100ull >> (8 * (31 - __clz(u | 1u)))) & 0xffu);
+  const int s = e + 127 - log2_pmax + ((b & 0x7fffffu) >= (u < 2u ? 0x800000u : 0x800000u - delta) ? 1 : 0);
+  return b - 1u < 0x7f7fffffu && s > 0 ? (uint32_t)s : 0u;
 }
 
 // E4M3 block scale code of a finite amax >= 0 (the P blocks), without a table or

@@ -352,11 +352,10 @@ mxfa_status mxfa_quantize_rows(const float* x, int64_t rows, int32_t cols, mxfa_
   if (!aligned16(x) || (reinterpret_cast<uintptr_t>(codes) & 3u))
     return fail(MXFA_ERR_INVALID_ARG, "x must be 16-byte and codes 4-byte aligned");
   int64_t nblocks = rows * (int64_t)cols / 32;
-  int64_t threads = nblocks * 8;
-  if (mxfa_status st = check_grid((threads + 255) / 256, 256)) return st;
+  if (mxfa_status st = check_grid((nblocks * 8 + 255) / 256, 256)) return st;
   DeviceModule* dm;
   if (mxfa_status st = module_for_current(&dm)) return st;
-  dim3 grid((unsigned)((threads + 255) / 256));
+  dim3 grid((unsigned)((nblocks + 127) / 128));   // 128 blocks per workgroup
   void* args[] = {(void*)&x, &nblocks, &codes, &scales};
   return launch(dm, fmt == MXFA_FMT_E4M3 ? "mxfa_quant_rows_e4m3" : "mxfa_quant_rows_e3m2", grid, dim3(256), args, stream);
 }

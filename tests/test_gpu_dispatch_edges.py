@@ -122,3 +122,29 @@ def test_gemm_small_and_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_
         torch.cuda.synchronize()
         assert bool(torch.isfinite(outs[0]).all())
         assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 32), (127, 32), (128, 32), (129, 64), (33, 4128)])
+@pytest.mark.parametrize("fmt", [mxfa.FMT_E4M3, mxfa.FMT_E3M2])
+def test_quantize_rows_block_counts(rows, cols, fmt):
+    """Workgroups of 128 blocks, four per thread: one block, one short of, exactly and one past a
+    workgroup, and a last workgroup partly filled."""
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols))
+    codes, scales = mxfa.quantize_rows(x.to(DEV), fmt)
+    want, want_sc = O.quantize_rows(x.numpy(), fmt)
+    np.testing.assert_array_equal(np_(codes), want)
+    np.testing.assert_array_equal(np_(scales), want_sc)
+
+
+@pytest.mark.parametrize("mats,rows,cols", [(1, 32, 4), (3, 32, 36), (1, 96, 128), (2, 64, 132), (5, 32, 260)])
+@pytest.mark.parametrize("fmt", [mxfa.FMT_E4M3, mxfa.FMT_E3M2, mxfa.FMT_E3M2_BLK])
+def test_quantize_cols_column_counts(mats, rows, cols, fmt):
+    """Waves of 128 columns, four to a workgroup: a few columns, a whole wave, a few past it, and
+    workgroups whose last waves have nothing."""
+    x = torch.randn(mats, rows, cols, generator=torch.Generator().manual_seed(mats + rows + cols))
+    codes, scales = mxfa.quantize_cols(x.to(DEV), fmt)
+    want, want_sc = O.quantize_cols(x.numpy(), O.FMT_E4M3 if fmt == mxfa.FMT_E4M3 else O.FMT_E3M2)
+    if fmt == mxfa.FMT_E3M2_BLK:
+        want = mxfa.e3m2_to_blk(want)
+    np.testing.assert_array_equal(np_(codes), want)
+    np.testing.assert_array_equal(np_(scales), want_sc)
