@@ -19,6 +19,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <string_view>
 #include <unordered_map>
 
 #include "mxfa_args.h"
@@ -160,10 +161,15 @@ mxfa_status loaded_module_for_current(DeviceModule** out) {
   return MXFA_OK;
 }
 
+// (a hashed index: walking the two hundred names cost about a microsecond per launch)
 hipFunction_t fn_by_name(DeviceModule* dm, const char* name) {
-  for (int i = 0; i < kNumKernels; i++)
-    if (std::strcmp(kKernelNames[i], name) == 0) return dm->fn[i];
-  return nullptr;
+  static const std::unordered_map<std::string_view, int> index = [] {
+    std::unordered_map<std::string_view, int> m;
+    for (int i = 0; i < kNumKernels; i++) m.emplace(kKernelNames[i], i);
+    return m;
+  }();
+  const auto it = index.find(name);
+  return it == index.end() ? nullptr : dm->fn[it->second];
 }
 
 // MXFA_PREFILL_LDS_PAD=<bytes>: that much dynamic LDS added to every prefill launch, which

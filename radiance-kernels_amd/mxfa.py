@@ -65,6 +65,8 @@ def _need(t, dtype, shape, name):
     on (the kernels read through raw pointers: a host, short or strided tensor would be
     read out of bounds)."""
     import torch
+    if type(t) is torch.Tensor and t.dtype is dtype and t.shape == shape and t.is_cuda and t.is_contiguous():
+        return
     if not (isinstance(t, torch.Tensor) and t.is_cuda):
         raise MxfaError(1, f"{name} must be a CUDA tensor")
     if t.dtype != dtype:
@@ -153,7 +155,7 @@ def _check(st):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None        # (the argtypes convert)
 
 
 def _stream(stream):
@@ -164,9 +166,9 @@ def _stream(stream):
         # decode-batch GEMM would otherwise wait on)
         raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if raw is not None:
-            return ctypes.c_void_p(raw(torch._C._cuda_getDevice()))
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(stream if isinstance(stream, int) else stream.cuda_stream)
+            return raw(torch._C._cuda_getDevice())
+        return torch.cuda.current_stream().cuda_stream
+    return stream if isinstance(stream, int) else stream.cuda_stream
 
 
 def init():
