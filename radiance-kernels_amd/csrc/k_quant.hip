@@ -37,7 +37,7 @@ __device__ __forceinline__ float4 load_nt(const float4* p) {
 typedef int v4i_u4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // x: rows of `cols` floats, 32-blocks along the row. nblocks = rows * cols / 32.  Memory-bound: each
-// thread quantizes its 4 values of QR_G blocks, 32 blocks apart, all loads (non-temporal: x is
+// thread quantizes its 4 values of per_thread (QR_G, or 1 for a small x) blocks, 32 blocks apart, all loads (non-temporal: x is
 // read once) issued before the first result and before the E3M2 table is filled.  134 MB of x
 // (from the MALL): E3M2 53.9 -> 33.5 us against one block per thread and the table first, E4M3 28.8
 // either way; Q, K and V of 268 MB (from HBM; V block-packed) 81.0 -> 64.9 us, 5.1 TB/s moved.
@@ -45,14 +45,14 @@ constexpr int QR_G = 4;
 
 template <int FMT>
 __device__ void quant_rows_impl(const float* __restrict__ x, int64_t nblocks, uint8_t* __restrict__ codes,
-                                uint8_t* __restrict__ scales) {
+                                uint8_t* __restrict__ scales, int per_thread) {
   __shared__ uint8_t e3m2_tab[FMT == 0 ? 4 : E3M2_TAB_N];
-  const int64_t blk0 = (int64_t)blockIdx.x * (QR_G * 32) + (threadIdx.x >> 3);
+  const int64_t blk0 = (int64_t)blockIdx.x * (per_thread * 32) + (threadIdx.x >> 3);
   const int part = (int)(threadIdx.x & 7);
   float4 v[QR_G];
 #pragma unroll
   for (int g = 0; g < QR_G; g++) {
-    const int64_t blk = blk0 + 32 * g;
+    const int64_t blk = g < per_thread ? blk0 + 32 * g : nblocks;
     v[g] = blk < nblocks ? load_nt(reinterpret_cast<const float4*>(x) + blk * 8 + part) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
   if constexpr (FMT != 0) {
@@ -61,6 +61,7 @@ __device__ void quant_rows_impl(const float* __restrict__ x, int64_t nblocks, ui
   }
 #pragma unroll
   for (int g = 0; g < QR_G; g++) {
+    if (g >= per_thread) break;
     const int64_t blk = blk0 + 32 * g;
     const float a = max8(fmaxf(fmaxf(fabsf(v[g].x), fabsf(v[g].y)), fmaxf(fabsf(v[g].z), fabsf(v[g].w))));
     const uint32_t sc = scale_code(a, FMT == 0 ? 8 : 4);
@@ -73,12 +74,12 @@ __device__ void quant_rows_impl(const float* __restrict__ x, int64_t nblocks, ui
 }
 
 extern "C" __global__ void __launch_bounds__(256) mxfa_quant_rows_e4m3(const float* x, int64_t nblocks,
-                                                                       uint8_t* codes, uint8_t* scales) {
-  quant_rows_impl<0>(x, nblocks, codes, scales);
+                                                                       uint8_t* codes, uint8_t* scales, int per_thread) {
+  quant_rows_impl<0>(x, nblocks, codes, scales, per_thread);
 }
 extern "C" __global__ void __launch_bounds__(256) mxfa_quant_rows_e3m2(const float* x, int64_t nblocks,
-                                                                       uint8_t* codes, uint8_t* scales) {
-  quant_rows_impl<1>(x, nblocks, codes, scales);
+                                                                       uint8_t* codes, uint8_t* scales, int per_thread) {
+  quant_rows_impl<1>(x, nblocks, codes, scales, per_thread);
 }
 
 // Rule R4 (the reference's SIMT block quantizer), 32-blocks along each row; amax is the

@@ -361,8 +361,11 @@ mxfa_status mxfa_quantize_rows(const float* x, int64_t rows, int32_t cols, mxfa_
   if (mxfa_status st = check_grid((nblocks * 8 + 255) / 256, 256)) return st;
   DeviceModule* dm;
   if (mxfa_status st = module_for_current(&dm)) return st;
-  dim3 grid((unsigned)((nblocks + 127) / 128));   // 128 blocks per workgroup
-  void* args[] = {(void*)&x, &nblocks, &codes, &scales};
+  // four blocks per thread where x is large enough to fill the chip with them (16 MB), else one (512
+  // blocks: 2.6 against 3.6 us)
+  int per_thread = nblocks >= 131072 ? 4 : 1;
+  dim3 grid((unsigned)((nblocks + 32 * per_thread - 1) / (32 * per_thread)));
+  void* args[] = {(void*)&x, &nblocks, &codes, &scales, &per_thread};
   return launch(dm, fmt == MXFA_FMT_E4M3 ? "mxfa_quant_rows_e4m3" : "mxfa_quant_rows_e3m2", grid, dim3(256), args, stream);
 }
 
