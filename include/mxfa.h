@@ -145,7 +145,7 @@ mxfa_status mxfa_prefill(const mxfa_attn_params *p,
  * Calls with too few query rows to fill the chip and a long key range (1,024 visible keys or more,
  * and at most 32 query rows or more than 5,120 keys) split the range: the workspace then holds
  * partial results, and O differs from mxfa_prefill's by the order of fp32 additions (rel-L2 below
- * 1e-6; the P codes are the same).
+ * 2e-6; the P codes are the same).
  * *workspace_bytes = batch * num_kv_heads * seq_k * head_dim * (2, or 3 with MXFA_FMT_E3M2 V).  A
  * workspace smaller than the plan is MXFA_ERR_WORKSPACE.
  * Replaces the same reference entry point as mxfa_prefill (kernels/flash_attention_mx_gqa/
