@@ -161,7 +161,7 @@ mxfa_status loaded_module_for_current(DeviceModule** out) {
   return MXFA_OK;
 }
 
-// (a hashed index: walking the two hundred names cost about a microsecond per launch)
+// (a hashed index: walking the two hundred names cost half a microsecond per launch)
 hipFunction_t fn_by_name(DeviceModule* dm, const char* name) {
   static const std::unordered_map<std::string_view, int> index = [] {
     std::unordered_map<std::string_view, int> m;
