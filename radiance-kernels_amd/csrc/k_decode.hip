@@ -253,7 +253,7 @@ __device__ void decode_split_impl(const FaArgs& a) {
       float M = -INFINITY;
       for (int i = 0; i < nparts; i++) {
         const float* qml = reinterpret_cast<const float*>(sVs[hg * nparts + i]);
-        if (qml[2 * q + 1] > 0.0f) M = fmaxf(M, qml[2 * q]);
+        M = vmax(M, qml[2 * q]);
       }
       float L = 0.0f;
       float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -261,10 +261,8 @@ __device__ void decode_split_impl(const FaArgs& a) {
         const float mc = M * c;
         for (int i = 0; i < nparts; i++) {
           const float* qml = reinterpret_cast<const float*>(sVs[hg * nparts + i]);
-          const float li = qml[2 * q + 1];
-          if (!(li > 0.0f)) continue;
           const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(qml[2 * q], c, -mc));
-          L += li * w;
+          L += qml[2 * q + 1] * w;
           const float4 o4 = reinterpret_cast<const float4*>(sV[hg * nparts + i])[fi];
           acc.x += o4.x * w;
           acc.y += o4.y * w;
@@ -273,10 +271,10 @@ __device__ void decode_split_impl(const FaArgs& a) {
         }
       }
       float4 v;
-      v.x = L > 0.0f ? acc.x / L : 0.0f;
-      v.y = L > 0.0f ? acc.y / L : 0.0f;
-      v.z = L > 0.0f ? acc.z / L : 0.0f;
-      v.w = L > 0.0f ? acc.w / L : 0.0f;
+      v.x = L != 0.0f ? acc.x / L : 0.0f;
+      v.y = L != 0.0f ? acc.y / L : 0.0f;
+      v.z = L != 0.0f ? acc.z / L : 0.0f;
+      v.w = L != 0.0f ? acc.w / L : 0.0f;
       const int b0 = bk0 / a.Hkv, kv0 = bk0 % a.Hkv;
       *reinterpret_cast<float4*>(a.o + ((int64_t)b0 * a.Hq + kv0 * G + q) * D + d) = v;
     }
@@ -327,6 +325,9 @@ MXFA_DECODE_ALL(128)
 MXFA_DECODE_ALL(256)
 
 // Merge nparts partials per (b, query head): O = sum_i O_i 2^{(m_i - M) c} / sum_i l_i 2^{(m_i - M) c}.
+// No partial is left out by its l: an empty one (m = -inf, O and l 0) has weight 0, and the NaN of
+// a NaN or infinite score (M by a maximum that keeps NaN) reaches its row as in one pass over the
+// keys.  A row without a visible key (M = -inf) is 0.
 // 16 lanes hold 64 columns of one partial (256 contiguous bytes).  One workgroup per (query head, 64
 // columns); group g = tid / 16 takes the partials g, g + ngrp, ... in order, CB_U of them in
 // flight (their loads issued before the maximum is known), and the groups' sums are added in
@@ -364,16 +365,13 @@ extern "C" __global__ void __launch_bounds__(512) mxfa_decode_combine(FaArgs a) 
   };
   load(grp);
   float M = -INFINITY;
-  for (int i = serial ? 0 : tid; i < nparts; i += serial ? 1 : blockDim.x) {
-    const float2 y = ml[i];
-    if (y.y > 0.0f) M = fmaxf(M, y.x);
-  }
+  for (int i = serial ? 0 : tid; i < nparts; i += serial ? 1 : blockDim.x) M = vmax(M, ml[i].x);
   if (!serial) {
 #pragma unroll
-    for (int k = 1; k < 64; k <<= 1) M = fmaxf(M, __shfl_xor(M, k));
+    for (int k = 1; k < 64; k <<= 1) M = vmax(M, __shfl_xor(M, k));
     if (lane == 0) smax[tid >> 6] = M;
     __syncthreads();
-    for (int w = 0; w < (int)blockDim.x >> 6; w++) M = fmaxf(M, smax[w]);
+    for (int w = 0; w < (int)blockDim.x >> 6; w++) M = vmax(M, smax[w]);
   }
   float L = 0.0f;
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -383,7 +381,7 @@ extern "C" __global__ void __launch_bounds__(512) mxfa_decode_combine(FaArgs a) 
       if (i0 != grp) load(i0);
 #pragma unroll
       for (int u = 0; u < CB_U; u++) {
-        if (i0 + u * ngrp < nparts && x[u].y > 0.0f) {
+        if (i0 + u * ngrp < nparts) {
           const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(x[u].x, c, -mc));
           L += x[u].y * w;
           acc.x += o[u].x * w;
@@ -395,7 +393,7 @@ extern "C" __global__ void __launch_bounds__(512) mxfa_decode_combine(FaArgs a) 
     }
   }
   if (serial) {
-    const bool any = L > 0.0f;
+    const bool any = L != 0.0f;
     *reinterpret_cast<float4*>(a.o + bh * D + d) = make_float4(any ? acc.x / L : 0.0f, any ? acc.y / L : 0.0f,
                                                                any ? acc.z / L : 0.0f, any ? acc.w / L : 0.0f);
     return;
@@ -409,6 +407,6 @@ extern "C" __global__ void __launch_bounds__(512) mxfa_decode_combine(FaArgs a) 
       s += so[g][tid];
       lt += sl[g];
     }
-    a.o[bh * D + 64 * blockIdx.y + tid] = lt > 0.0f ? s / lt : 0.0f;
+    a.o[bh * D + 64 * blockIdx.y + tid] = lt != 0.0f ? s / lt : 0.0f;
   }
 }

@@ -27,6 +27,50 @@ def test_nan_key_code_reaches_every_row_that_sees_it(D, softcap, ws):
     assert bool(nan[:, 128:].all()) and bool(torch.isfinite(o[0, :, :100]).all())
 
 
+@pytest.mark.parametrize("v_fmt", [mxfa.FMT_E4M3, mxfa.FMT_E3M2, mxfa.FMT_E3M2_BLK])
+@pytest.mark.parametrize("D,softcap,p_rule", [(64, 0.0, mxfa.P_R1), (128, 0.0, mxfa.P_R1), (128, 30.0, mxfa.P_R1),
+                                              (256, 30.0, mxfa.P_R1), (256, 0.0, mxfa.P_R2)])
+@pytest.mark.parametrize("where,pos", [("key", 5), ("key", 1000), ("key", 1997), ("scale", 700), ("query", 3),
+                                       ("infinite", 600)])
+def test_nan_and_infinite_scores_pass_the_split_merge(D, softcap, p_rule, v_fmt, where, pos):
+    """A split call (32 key blocks) with a NaN code in the first, a middle or the last key range, a NaN
+    scale, a NaN query code or scores that overflow: the rows of mxfa_prefill (one pass) that are
+    NaN are NaN, and only they."""
+    n = 2000
+    _, dev, _ = gen_qkv(1, 4, 2, 8, 2016, D, seed=78, v_fmt=v_fmt)
+    if where == "key":
+        dev["k"][0, 1, pos, 3] = 0x7F
+    elif where == "scale":
+        dev["ks"][0, 1, pos, 0] = 255
+    elif where == "query":
+        dev["q"][0, 2, pos, 1] = 0x7F
+    else:                                                  # 448 x 2^127 per product
+        dev["ks"][0, 1, pos] = 254
+        dev["k"][0, 1, pos] = 0x7E
+    p = mxfa.make_params(1, 4, 2, 8, 2016, D, causal=True, q_pos0=n - 8, softcap=softcap, v_fmt=v_fmt, p_rule=p_rule)
+    ops = [dev[x] for x in ("q", "qs", "k", "ks", "v", "vs")]
+    split = torch.isnan(mxfa.prefill(p, *ops))
+    one = torch.isnan(mxfa.prefill(p, *ops, workspace=False))
+    torch.cuda.synchronize()
+    assert bool(one.any())
+    assert torch.equal(split, one)
+
+
+@pytest.mark.parametrize("waves,combine", [(1, None), (2, None), (4, None), (4, "kernel"), (24, None), (200, None)])
+def test_nan_key_code_reaches_the_decoded_row(monkeypatch, waves, combine):
+    """Merged inside the workgroup or by mxfa_decode_combine, a partial with a NaN is not left out."""
+    monkeypatch.setenv("MXFA_DECODE_WAVES", str(waves))
+    if combine:
+        monkeypatch.setenv("MXFA_DECODE_COMBINE", combine)
+    L = 64 * 200
+    _, dev, _ = gen_qkv(1, 4, 2, 1, L, 128, seed=79)
+    dev["k"][0, 1, 5000, 3] = 0x7F
+    p = mxfa.make_params(1, 4, 2, 1, L, 128, causal=True, q_pos0=L - 5)
+    o = mxfa.decode(p, *(dev[x] for x in ("q", "qs", "k", "ks", "v", "vs")))
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(o[0, 2:]).all()) and bool(torch.isfinite(o[0, :2]).all())
+
+
 @pytest.mark.parametrize("parts", [4, 5, 16, 17, 32, 33, 128, 129, 257, 300])
 def test_decode_merge_part_counts(monkeypatch, parts):
     """mxfa_decode_combine at the edges of its part groups: one up to 4 partials, then 4, 16 and 32
