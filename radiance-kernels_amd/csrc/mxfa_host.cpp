@@ -640,6 +640,25 @@ size_t prefill3_workspace(const mxfa_attn_params* p) {
   return prefill3_kbf_bytes(p) + v;
 }
 
+// Whether n ranges of a call's `longest` key blocks take less time than one walk over them, by an
+// estimate in us fitted to 1,377 calls (D = 64, 128, 256; 1 to 512 rows, batch 1 to 64, 1,000 to 32,768
+// keys), each timed both ways: a block takes `block` in a workgroup that has its CU nearly to
+// itself; one walk slows down by 0.9 per workgroup and CU, n ranges by `share` (their waves hide
+// each other's latency); the maxima add a third; two more launches and the ramp cost 8 us, the
+// partials 3 MB per us written and read.  Of the 1,133 calls that the other rules split it leaves
+// out 51: 40 are slower split (1.9 times at most), 5 gain more than 4% (13% at most).  Of the calls
+// still split the worst loses 4%.
+bool split_pays(const mxfa_attn_params* p, int64_t items, int longest, int n, int64_t partial_bytes) {
+  const double block = (p->head_dim == 256 ? 2.8 : p->head_dim == 128 ? 1.8 : 1.3) *
+                       (1.0 + (p->softcap > 0.0f ? 0.3 : 0.0) + (p->p_rule == MXFA_P_R2 ? 0.15 : 0.0));
+  const double share = p->head_dim == 256 ? 0.8 : p->head_dim == 128 ? 0.6 : 0.5;
+  const double per_cu = items / 256.0;
+  const double one = block * longest * std::max(1.0, 0.9 * per_cu);
+  const double split = 8.0 + 4.0 / 3.0 * block * ((longest + n - 1) / n) * std::max(1.0, share * per_cu * n) +
+                       2.0 * partial_bytes / 3e6;
+  return split < one;
+}
+
 // Key ranges per query block of a mxfa_prefill_ws call (1: not split).  A few rows against a long
 // cache (a prompt chunk, drafted tokens to verify) give a grid of `items` workgroups that leaves
 // most of the chip idle for the whole walk over the keys.  Split, three launches: the row maxima
@@ -663,7 +682,11 @@ size_t prefill3_workspace(const mxfa_attn_params* p) {
 // - from 16 visible key blocks on (8 rows; 8 blocks: 20 -> 18 us only), and for more than one query
 //   tile per head (32 rows) in calls of more than 5,120 keys: shorter ones keep their
 //   bit-identity with mxfa_prefill, at the price of what 64 rows x 4,096 keys could gain (103 ->
-//   40 us).
+//   40 us);
+// - where the split is estimated to be the faster form (split_pays): many rows over a short range
+//   spend more on writing and merging the partials than the shorter walk saves (batch 32 of 32
+//   rows x 1,000 keys, D = 64: 26 -> 51 us split; batch 24, D = 128: 39 -> 60; batch 20, D = 256:
+//   50 -> 77).
 int prefill_splits(const FaArgs& a, const mxfa_attn_params* p, int64_t items) {
   const int64_t slots = p->head_dim == 256 ? 512 : p->head_dim == 128 ? 768 : 1024;
   const int nkb = (p->seq_k + 63) / 64;
@@ -678,7 +701,7 @@ int prefill_splits(const FaArgs& a, const mxfa_attn_params* p, int64_t items) {
   const int64_t row_bytes = (int64_t)p->batch * p->num_q_heads * p->seq_q * (p->head_dim + 3) * (int64_t)sizeof(float);
   int64_t n = std::min(slots / items, (int64_t)std::sqrt(8.0 * longest));
   n = std::min(n, (int64_t)prefill3_workspace(p) / row_bytes);
-  return n >= 3 || (n == 2 && items <= 128) ? (int)n : 1;
+  return (n >= 3 || (n == 2 && items <= 128)) && split_pays(p, items, longest, (int)n, n * row_bytes) ? (int)n : 1;
 }
 
 }  // namespace

@@ -127,6 +127,23 @@ def test_split_prefill_matches_single_pass(B, Hq, Hkv, Sq, n, D, kw):
     assert rel <= 2e-6
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,n,D,kw", [
+    (32, 32, 8, 32, 1000, 64, {}),
+    (24, 32, 8, 32, 1500, 128, dict(window=1300)),
+    (20, 32, 8, 32, 1000, 256, dict(softcap=30.0, p_rule=mxfa.P_R2)),
+])
+def test_short_prefill_of_many_rows_is_one_pass(B, Hq, Hkv, Sq, n, D, kw):
+    """Where the partials of a split would cost more than the shorter walk saves, mxfa_prefill_ws runs
+    the single pass: bit-identical with mxfa_prefill."""
+    Sk = (n + 31) // 32 * 32
+    _, dev, _ = gen_qkv(B, Hq, Hkv, Sq, Sk, D, seed=400 + n)
+    p = mxfa.make_params(B, Hq, Hkv, Sq, Sk, D, causal=True, q_pos0=n - Sq, **kw)
+    ops = [dev[x] for x in ("q", "qs", "k", "ks", "v", "vs")]
+    ws, one = mxfa.prefill(p, *ops), mxfa.prefill(p, *ops, workspace=False)
+    torch.cuda.synchronize()
+    assert torch.equal(ws, one)
+
+
 @pytest.mark.parametrize("M,N,K,a_fmt,b_fmt", [
     # 64 x 64 tiles (256 k per stage)
     (48, 64, 64, 0, 0),              # one half: no whole stage
