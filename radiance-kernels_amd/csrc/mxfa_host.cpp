@@ -361,9 +361,11 @@ mxfa_status mxfa_quantize_rows(const float* x, int64_t rows, int32_t cols, mxfa_
   if (mxfa_status st = check_grid((nblocks * 8 + 255) / 256, 256)) return st;
   DeviceModule* dm;
   if (mxfa_status st = module_for_current(&dm)) return st;
-  // four blocks per thread where x is large enough to fill the chip with them (16 MB), else one (512
-  // blocks: 2.6 against 3.6 us)
-  int per_thread = nblocks >= 131072 ? 4 : 1;
+  // One block per thread for a small x, four where there are enough of them to fill the chip.  us for
+  // one and four, x from the MALL (from HBM): E4M3 131,072 blocks 6.4 and 6.9 (6.1 and 6.4), 230,000 9.1
+  // and 10.1 (8.8 and 9.6), 524,288 16.5 and 16.3 (17.2 and 17.3); E3M2, whose table each workgroup
+  // fills once, 131,072 9.6 and 8.4 (9.1 and 7.7).
+  int per_thread = nblocks >= (fmt == MXFA_FMT_E4M3 ? 524288 : 131072) ? 4 : 1;
   dim3 grid((unsigned)((nblocks + 32 * per_thread - 1) / (32 * per_thread)));
   void* args[] = {(void*)&x, &nblocks, &codes, &scales, &per_thread};
   return launch(dm, fmt == MXFA_FMT_E4M3 ? "mxfa_quant_rows_e4m3" : "mxfa_quant_rows_e3m2", grid, dim3(256), args, stream);

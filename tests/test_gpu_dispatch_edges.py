@@ -185,11 +185,12 @@ def test_gemm_small_and_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_
         assert torch.equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 32), (31, 32), (33, 64), (131071, 32), (131072, 32), (131073, 32), (1025, 4128)])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (31, 32), (33, 64), (131071, 32), (131072, 32), (131073, 32), (1025, 4128),
+                                       (4096, 4064), (4096, 4096), (4097, 4128)])
 @pytest.mark.parametrize("fmt", [mxfa.FMT_E4M3, mxfa.FMT_E3M2])
 def test_quantize_rows_block_counts(rows, cols, fmt):
-    """Workgroups of 32 blocks, or of 128 (four per thread) from 131,072 blocks on: around both
-    workgroup sizes and the change between them."""
+    """Workgroups of 32 blocks, or of 128 (four per thread) from 131,072 blocks (E3M2) or 524,288
+    (E4M3) on: around both workgroup sizes and the change between them."""
     x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols))
     codes, scales = mxfa.quantize_rows(x.to(DEV), fmt)
     want, want_sc = O.quantize_rows(x.numpy(), fmt)
