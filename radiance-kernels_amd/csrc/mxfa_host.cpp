@@ -306,12 +306,14 @@ int decode_parts_max(const mxfa_attn_params* p) {
 // Of those, no more than the blocks that the query sees: with a window in a longer cache the other
 // partials are empty (window 4,096 in a cache of 60,000 keys: 65 of 938 blocks visible, 256 partials
 // 14.1 us a call, 65 12.6).  Each visible block is then a partial of its own in either plan, so O
-// differs by the order of the merge's fp32 sums only.  (Fewer partials than that can be faster
+// differs by the order of the merge's fp32 sums only.  Not where a head's partials share a workgroup
+// at D = 256 (one workgroup per CU) in any case: fewer of them only put the visible blocks on fewer
+// CUs (batch 32, Hkv 8, 2 blocks visible: 11.6 us in 4 partials, 12.9 in 2).  (Fewer partials than that can be faster
 // -- 96 heads of 47 blocks at D = 256, 264 workgroups on 256 CUs in 11 partials each: 50.2 us, in 10
 // 32.7 -- but change the running maxima that P is quantized against.)
 int decode_parts(const mxfa_attn_params* p) {
   const int nmax = decode_parts_max(p);
-  if (p->window <= 0 || decode_wave_override()) return nmax;
+  if (p->window <= 0 || decode_wave_override() || (p->head_dim == 256 && nmax <= 4)) return nmax;
   const int hi = p->causal ? std::min(p->seq_k - 1, p->q_pos0) : p->seq_k - 1;
   const int lo = std::max(0, p->q_pos0 - p->window + 1);
   const int vis = hi >= lo ? hi / 64 - lo / 64 + 1 : 1;

@@ -24,3 +24,18 @@ def test_workspace_covers_shorter_caches(monkeypatch):
         assert B * Hkv * group * parts * (D + 2) * 4 <= ws
         visible = min(n, window) if window else n
         assert 1 <= parts <= max(4, (visible + 63) // 64 + 1)
+
+
+def test_partials_that_share_a_workgroup_stay_spread_at_d256(monkeypatch):
+    """At D = 256 (one workgroup per CU) a plan of up to 4 partials keeps them with a window: in fewer the
+    visible blocks would sit on fewer CUs.  At D = 128 (two workgroups per CU) and in larger plans the
+    window still limits them."""
+    monkeypatch.delenv("MXFA_DECODE_WAVES", raising=False)
+    for B, parts in ((32, 4), (64, 2)):
+        for n in (500, 3000):
+            assert _plan(B, 8, 4, n, 256, 0)[0] == parts
+            assert _plan(B, 8, 4, n, 256, 100)[0] == parts
+    assert _plan(64, 8, 4, 3000, 128, 0)[0] == 4
+    assert _plan(64, 8, 4, 3000, 128, 100)[0] == 2
+    assert _plan(8, 8, 4, 3000, 256, 0)[0] == 16
+    assert _plan(8, 8, 4, 3000, 256, 100)[0] == 2
