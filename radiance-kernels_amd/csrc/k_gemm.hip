@@ -824,11 +824,11 @@ __device__ __forceinline__ v4i rsrc_words(const uint8_t* base, int64_t off, int6
 }
 __device__ __forceinline__ void dma_asm16(v4i rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
   __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
 }
 __device__ __forceinline__ void dma_asm4(v4i rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
   __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+                   : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0", "memory");
 }
 
 template <int TI, int TJ, int NSUB> struct GdmaCfg {
