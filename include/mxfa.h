@@ -142,10 +142,13 @@ mxfa_status mxfa_prefill(const mxfa_attn_params *p,
  * inputs, outputs and O as mxfa_prefill (bit-identical with E4M3 V, where both run the same
  * arithmetic in the same order; within a few ulps with E3M2 V).  Block-packed E3M2 V needs no
  * copy: the kernel reads it from v as it is.
- * Calls with too few query rows to fill the chip and a long key range (1,024 visible keys or more,
- * and at most 32 query rows or more than 5,120 keys) split the range: the workspace then holds
- * partial results, and O differs from mxfa_prefill's by the order of fp32 additions (rel-L2 below
- * 2e-6; the P codes are the same).
+ * Calls with too few query rows to fill the chip and a long key range (16 or more 64-key blocks
+ * that some query row's workgroup reads -- a block counts from its first visible key on, so 961
+ * keys can be enough -- and at most 32 query rows or seq_k above 5,120) may split the range, where
+ * that is estimated to be the faster form: the workspace then holds partial results, and O differs
+ * from mxfa_prefill's by the order of fp32 additions; the P codes are the same, and a row that is
+ * NaN there is NaN here.  Measured rel-L2 of the difference: below 2e-6 up to 300,000 keys, 2.7e-6
+ * at 524,288 and 1.3e-5 at 8,000,000, where most of it is the rounding of the single pass's own sums.
  * *workspace_bytes = batch * num_kv_heads * seq_k * head_dim * (2, or 3 with MXFA_FMT_E3M2 V).  A
  * workspace smaller than the plan is MXFA_ERR_WORKSPACE.
  * Replaces the same reference entry point as mxfa_prefill (kernels/flash_attention_mx_gqa/

@@ -669,7 +669,8 @@ bool split_pays(const mxfa_attn_params* p, int64_t items, int longest, int n, in
 // of every range but the last (prefill_max_impl), the attention kernel per range, starting from
 // the maximum of the ranges before it -- so every P and its code are the unsplit call's -- and
 // the merge of the partials.  O differs from the unsplit call's by the order of fp32 sums only
-// (3e-7 rel-L2 at most over 60 random calls).  Measured, unsplit -> split (ranges):
+// (rel-L2 3e-7 at most over 60 random calls, 6e-7 at 131,072 keys in 128 ranges, 1.3e-5 at 8,000,000 in
+// 1,000).  Measured, unsplit -> split (ranges):
 //   Hq 32, Hkv 8, D = 128:  200 rows x 32,768 keys 1,009 -> 207 us (13), 8 x 8,192 254 -> 28 (32),
 //     8 x 1,024 36 -> 18 (11), batch 8 of 8 x 4,096 131 -> 47 (12), 512 x 16,384 391 -> 258 (3)
 //   Hq 16, Hkv 8, D = 256:  256 x 16,384 631 -> 123 (16), 30 x 2,048 softcap 111 -> 30 (16), 256 x

@@ -127,6 +127,29 @@ def test_split_prefill_matches_single_pass(B, Hq, Hkv, Sq, n, D, kw):
     assert rel <= 2e-6
 
 
+@pytest.mark.parametrize("Hq,Hkv,Sq,n,D,v_fmt,ranges", [
+    (2, 1, 8, 20000, 64, mxfa.FMT_E4M3, 50),                    # merged by 16 groups
+    (4, 1, 5, 131072, 128, mxfa.FMT_E3M2_BLK, 128),             # the most of them
+    (2, 1, 8, 160000, 64, mxfa.FMT_E3M2, 141),                  # 32 groups
+    (2, 1, 3, 300000, 256, mxfa.FMT_E4M3, 193),
+])
+def test_split_prefill_of_many_ranges(Hq, Hkv, Sq, n, D, v_fmt, ranges):
+    """As above for long caches: sqrt(8 x key blocks) ranges.  Every range is rounded once more in the
+    merge (2^-24 of the row), and both passes round their own sums over the blocks, independently
+    (the root of their number)."""
+    Sk = (n + 31) // 32 * 32
+    _, dev, _ = gen_qkv(1, Hq, Hkv, Sq, Sk, D, seed=500 + n // 1000, v_fmt=v_fmt)
+    p = mxfa.make_params(1, Hq, Hkv, Sq, Sk, D, causal=True, q_pos0=n - Sq, v_fmt=v_fmt)
+    ops = [dev[x] for x in ("q", "qs", "k", "ks", "v", "vs")]
+    ws = torch.full((mxfa.prefill_plan(p),), 255, dtype=torch.uint8, device=DEV)
+    split, one = mxfa.prefill(p, *ops, workspace=ws), mxfa.prefill(p, *ops, workspace=False)
+    torch.cuda.synchronize()
+    assert not torch.equal(split, one), "the call was not split"
+    rel, _ = errors(np_(split), np_(one))
+    print(f"   {ranges} ranges against one pass: rel-L2 {rel:.3e}", flush=True)
+    assert rel <= (ranges + (Sk / 64) ** 0.5) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,n,D,kw", [
     (32, 32, 8, 32, 1000, 64, {}),
     (24, 32, 8, 32, 1500, 128, dict(window=1300)),
