@@ -361,8 +361,8 @@ def bench_gemm(torch, mxfa, args):
     c16 = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     ms16 = time_calls(torch, lambda: mxfa.gemm(xq, xs, wq, ws, out=c16, c_fmt=mxfa.C_BF16), args.steps, args.warmup)
     tf16 = 2.0 * M * N * K / (ms16 * 1e-3) / 1e12
-    # the same weights at decode batch M = 64 (the skinny kernel: one workgroup per 32-column
-    # strip); HBM-bound on the weights, so reported as the weight stream rate
+    # the same weights at decode batch M = 64 (64 x 64 tiles, 96 workgroups), reported as the
+    # rate at which the weights stream (repeated calls: from the last-level cache)
     Md = 64
     Xd = torch.empty((Md, K), dtype=torch.float32, device=dev)
     mxfa.fill_normal(Xd, 43)

@@ -8,6 +8,7 @@ torch = pytest.importorskip("torch")
 import mxfa  # noqa: E402
 import oracle as O  # noqa: E402
 from gpuhelp import DEV, MAX_ABS_TOL, REL_L2_TOL, errors, gen_qkv, np_, oracle_params  # noqa: E402
+from test_gpu_gemm import run_gemm  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -206,6 +207,45 @@ def test_gemm_small_and_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_
         torch.cuda.synchronize()
         assert bool(torch.isfinite(outs[0]).all())
         assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("M,N,K,strips", [
+    (16, 48, 8256, True), (32, 8192, 1088, True),                # M <= 32: up to 256 strips of 32 columns
+    (32, 8208, 1088, False),
+    (48, 80, 8256, True), (64, 4096, 14336, True),               # M <= 64: K above 8,192; 129 steps of 64 k, half a strip
+    (64, 8192, 8256, True), (64, 8208, 8256, False),
+    (64, 96, 8192, False),
+    (64, 96, 32768, True), (64, 96, 32832, False),               # the scales fill the strip kernel's LDS exactly; past it
+    (80, 96, 8256, False),
+])
+def test_gemm_strip_kernel_dispatch(monkeypatch, M, N, K, strips):
+    """The k-split strip kernel on its side of each line of the dispatch and the tiles (C bit-identical with
+    the 256 x 256 kernels) on the other.  Against the 256 x 256 kernels the strips add the same
+    products in another order: as in test_gemm_skinny_matches_oracle_and_tiled_kernel, whose
+    bound is 2^-12 of the terms' absolute sum; with terms of random sign that sum is about the
+    root of K times the result, 2^-12 sqrt(K) of it at most."""
+    monkeypatch.delenv("MXFA_GEMM", raising=False)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M + N + K)
+    a, b = (torch.randint(0, 256, shape, generator=g, device=DEV, dtype=torch.int32) for shape in ((M, K), (K, N)))
+    a, b = (torch.where((c & 127) == 127, c - 1, c).to(torch.uint8) for c in (a, b))
+    sa, sb = (torch.randint(112, 142, (K // 32, n), generator=g, device=DEV, dtype=torch.int32).to(torch.uint8) for n in (M, N))
+    c, again = mxfa.gemm(a, sa, b, sb), mxfa.gemm(a, sa, b, sb)
+    c16 = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    mxfa.gemm(a, sa, b, sb, out=c16, c_fmt=mxfa.C_BF16)
+    monkeypatch.setenv("MXFA_GEMM", "big")
+    big = mxfa.gemm(a, sa, b, sb)
+    torch.cuda.synchronize()
+    assert torch.equal(c, again) and torch.equal(c16, c.to(torch.bfloat16))
+    assert torch.equal(c, big) != strips
+    rel, _ = errors(np_(c), np_(big))
+    assert rel <= 2.0 ** -12 * K ** 0.5
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 80, 8256), (64, 208, 14336), (64, 48, 9216)])
+def test_gemm_two_tile_strip_kernel_matches_oracle(M, N, K):
+    """33 to 64 rows on the strip kernel, within the oracle's bound of every mxfa_gemm."""
+    run_gemm(M, N, K, seed=M + N + K)
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 32), (31, 32), (33, 64), (131071, 32), (131072, 32), (131073, 32), (1025, 4128),

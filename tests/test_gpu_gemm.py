@@ -53,9 +53,9 @@ def test_gemm_matches_oracle(M, N, K):
 @pytest.mark.parametrize("i", sweep_seeds(range(12), "MXFA_GEMM_SEEDS"))
 def test_gemm_sweep(i, monkeypatch):
     """Seeded shapes (M = 16 .. 1,024, N = 16 .. 1,104, K = 64 .. 2,496) with E4M3 or E3M2
-    operands through each kernel path (the default choice -- skinny for M <= 128, else the
-    LDS-DMA kernel for E4M3 with K % 128 == 0 -- MXFA_GEMM=big or =reg); MXFA_GEMM_SEEDS=0-300
-    runs the exploratory length."""
+    operands through the default choice (the strip kernel for M <= 32, 64 x 64 or 128 x 128 tiles
+    otherwise: E3M2 operands always the latter) or MXFA_GEMM=big or =reg; MXFA_GEMM_SEEDS=0-300 runs
+    the exploratory length."""
     rng = np.random.default_rng(31000 + i)
     M = 16 * int(rng.choice([1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 33, 64]))
     N = 16 * int(rng.integers(1, 70))
@@ -179,10 +179,11 @@ def test_gemm_dma_kernel_equals_register_staged(monkeypatch, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(16, 64, 64), (32, 96, 1024), (48, 80, 192), (64, 6144, 4096), (96, 208, 576),
                                    (128, 512, 2048), (112, 48, 4160)])
 def test_gemm_skinny_matches_oracle_and_tiled_kernel(monkeypatch, M, N, K):
-    """M <= 128 with E4M3 operands runs the skinny kernel (one workgroup per 32-column strip, the
-    64-k steps split over its four waves, partials summed in wave order): within the oracle's
-    bound like every mxfa_gemm, close to the tiled kernel (MXFA_GEMM=big: the same products,
-    accumulated in another order), deterministic, fp32 and bf16 C."""
+    """Small M with E4M3 operands.  M <= 32 runs the strip kernel (one workgroup per 32-column strip, the
+    64-k steps split over its four waves, partials summed in wave order), the other shapes the
+    64 x 64 tiles (above M = 32 the strips need K > 8,192: test_gemm_strip_kernel_dispatch).  Within
+    the oracle's bound like every mxfa_gemm, close to the 256 x 256 kernel (MXFA_GEMM=big: the same
+    products, by the strips accumulated in another order), deterministic, fp32 and bf16 C."""
     print(f"skinny gemm M{M} N{N} K{K}", flush=True)
     rng = np.random.default_rng(M * 7 + N + K)
     a, b = _codes(rng, (M, K), 0), _codes(rng, (K, N), 0)
