@@ -788,16 +788,10 @@ __device__ __forceinline__ void gemm_mid_impl(const GemmArgs& g) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  constexpr int U = 2 * R / (R % 2 ? 1 : 2);          // slots and stages repeat every U steps
-  for (int kt = 0; kt < nk; kt += U) {
+  static_assert(R == 2, "slots and LDS stages repeat every two steps");
+  for (int kt = 0; kt < nk; kt += 2) {
     step(std::integral_constant<int, 0>{}, kt);
     if (kt + 1 < nk) step(std::integral_constant<int, 1>{}, kt + 1);
-    if constexpr (U > 2) {
-      if (kt + 2 < nk) step(std::integral_constant<int, 2>{}, kt + 2);
-      if (kt + 3 < nk) step(std::integral_constant<int, 3>{}, kt + 3);
-      if (kt + 4 < nk) step(std::integral_constant<int, 4>{}, kt + 4);
-      if (kt + 5 < nk) step(std::integral_constant<int, 5>{}, kt + 5);
-    }
   }
   __syncthreads();
 
@@ -858,7 +852,7 @@ __device__ __forceinline__ void gdma_read(GdmaOps<TI, TJ>& o, const uint8_t* sub
   const uint8_t *sB = sub + C::A_BYTES, *sSA = sB + C::B_BYTES, *sSB = sSA + C::SA;
 #pragma unroll
   for (int j = 0; j < TJ; j++) {
-    if (j != p * TJ / (TI * TJ) || p * TJ % (TI * TJ) != 0) continue;
+    if (TI * j != p) continue;
     const int ncol = 32 * TJ * wc + 32 * j + 16 * (g16 & 1) + 8 * (l16 & 1);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
