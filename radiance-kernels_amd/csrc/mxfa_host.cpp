@@ -512,10 +512,13 @@ mxfa_status mxfa_gemm(const mxfa_gemm_params* p, const uint8_t* a, const uint8_t
   const bool e4m3 = !g.a_e3m2 && !g.b_e3m2;
   // M <= 64 with E4M3 operands (the batched-decode projection): the skinny kernel, one workgroup per
   // 32-column strip (its LDS holds all of SA and the strip's SB: (k / 32) (m + 32) <= 96 KiB), while
-  // the strips fit the chip at once (N = 14,336, M = 64: 28 us, the tiles below 16) and, above M =
-  // 32, only for a long K (us at K = 4,096, N = 6,144, skinny and 64 x 64 tiles: M = 16 11.4 and 12.2,
-  // 32 12.4 and 12.5, 64 14.8 and 13.4; K = 14,336, N = 4,096: 30.6 and 35.1, 32.0 and 36.4, 38.9 and
-  // 40.7; K = 7,168, N = 2,048, M = 64 13.2 and 10.6).
+  // the strips fit the chip at once (us, strips and 64 x 64 tiles, weights from HBM: N = 10,240, K = 512
+  // M = 16 8.8 and 5.0, M = 32 9.3 and 5.2; K = 4,096 32.3 and 22.8, 34.1 and 23.6; K = 14,336 89 and 72,
+  // 93 and 77) and, above M = 32, only for a long K.  Up to there the tiles are faster on weights that
+  // the caches hold and the strips on weights from HBM (us, M = 64, N = 4,096: K = 4,096 11.2 and 7.6
+  // cached, 21.0 and 20.8 from HBM; 6,144 13.9 and 9.4, 28.2 and 30.3; 8,192 23.1 and 22.4, 35.5 and
+  // 38.5; N = 2,048, K = 8,192 18.9 and 14.6, 34.4 and 39.1), above it the strips either way (K =
+  // 14,336, N = 4,096, cached: M = 16 30.6 and 35.1, 32 32.0 and 36.4, 64 38.9 and 40.7).
   const int64_t strips = (p->n + 31) / 32;
   if (e4m3 && p->m <= 64 && (p->k / 32) * (p->m + 32) <= 96 * 1024 && strips <= 256 && (p->m <= 32 || p->k > 8192) &&
       !selected("big") && !selected("reg") && !selected("mid")) {
