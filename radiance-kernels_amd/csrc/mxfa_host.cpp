@@ -539,11 +539,15 @@ mxfa_status mxfa_gemm(const mxfa_gemm_params* p, const uint8_t* a, const uint8_t
   // rounds over the CUs and the smaller ones at most twice as many: a K step of 128 takes 0.3 us
   // against 1.1.  N = 6,144, K = 4,096: M = 400 16 against 43 us, 1,024 (384 tiles of 128) 36 against
   // 44; 2,048 (768, three rounds against one) 57 against 47.  With E3M2 operands (two workgroups
-  // per CU): M = 400 35 against 69 us, 1,024 50 against 69.
+  // per CU): M = 400 35 against 69 us, 1,024 50 against 69.  A second round of them pays from k = 1,024
+  // on, or where the 256 x 256 tiles would be the register-staged ones (k % 128 = 64): M = 1,024, N =
+  // 6,144, 256 and 128 tiles: k = 128 8.8 and 10.1 us, 192 12.6 and 10.2, 384 11.1 and 11.8, 768 16.2 and
+  // 17.3, 1,024 20.0 and 20.6, 2,048 34.0 and 31.9; N = 5,120 1,024 19.7 and 19.1.
   const int64_t tiles128 = (p->m + 127) / 128 * ((p->n + 127) / 128);
   const int64_t rounds256 = (tm * tn + 255) / 256;
   if (selected("mid") || (!sel && rounds256 <= 2 &&
-                          (e4m3 ? (tiles128 + 255) / 256 <= 2 * rounds256 : (tiles128 + 511) / 512 <= rounds256))) {
+                          (e4m3 ? tiles128 <= 256 || ((p->k >= 1024 || p->k % 128) && (tiles128 + 255) / 256 <= 2 * rounds256)
+                                : (tiles128 + 511) / 512 <= rounds256))) {
     g.tiles_n = (int)((p->n + 127) / 128);
     const char* mid = e4m3         ? "mxfa_gemm_mid_dma"
                       : !g.a_e3m2  ? "mxfa_gemm_mid_be3m2"

@@ -180,6 +180,8 @@ def test_short_prefill_of_many_rows_is_one_pass(B, Hq, Hkv, Sq, n, D, kw):
     (160, 6160, 192, 0, 0),          # a step and a half, columns and rows past the tile
     (400, 4112, 576, 0, 0),          # 4 whole steps and a half, ragged
     (1024, 4096, 640, 0, 0),         # 256 tiles
+    (1024, 4112, 448, 0, 0),         # a second round of tiles: K % 128 = 64 (256 x 256 tiles below K = 1,024 otherwise)
+    (1024, 4112, 896, 0, 0), (1040, 4096, 1024, 0, 0),
     (272, 272, 1088, 0, 1), (256, 144, 64, 1, 0), (48, 400, 320, 1, 1),
 ])
 def test_gemm_small_and_mid_tiles_equal_register_staged(monkeypatch, M, N, K, a_fmt, b_fmt):
